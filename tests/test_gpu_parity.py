@@ -163,6 +163,31 @@ def test_absmax_quantizers(gpu, k):
         assert same_bits(host(ds2, np.float32, m)[r:r + 1], np.float32([s2]))
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("k", [1, 3, 31, 32, 33, 2047, 2048, 2049, 4100, 6911])
+def test_subln_absmax_sizes(gpu, k, offset):
+    """The ordered sum of squares around its 32-value reads and 2048-value LDS buffers, and rows that
+    are not 16-byte aligned; an Inf and a NaN row."""
+    torch = gpu
+    rng = np.random.default_rng(k + offset)
+    m = 3
+    x = (rng.standard_normal((m, k)) * rng.choice([1e-3, 1, 50], (m, k))).astype(np.float32)
+    x[1, k // 2], x[2, 0] = np.inf, np.nan
+    w = rng.uniform(-1.5, 1.5, k).astype(np.float32)
+    dx = torch.zeros(m * k + 4, dtype=torch.float32, device="cuda")
+    dx[offset:offset + m * k] = torch.from_numpy(x.reshape(-1)).cuda()
+    dw = torch.zeros(k + 4, dtype=torch.float32, device="cuda")
+    dw[offset:offset + k] = torch.from_numpy(w).cuda()
+    dq, ds = empty(torch, m * k + 4), empty(torch, 4 * m)
+    jk.dev_subln_quantize_absmax_i8(dx[offset:], dw[offset:], m, k, 1e-5, dq[offset:], ds)
+    torch.cuda.synchronize()
+    got = host(dq, np.int8, m * k + 4)[offset:offset + m * k].reshape(m, k)
+    for r in range(m):
+        q, s = O.subln_quantize_absmax_i8(x[r], w, 1e-5)
+        assert np.array_equal(got[r], q)
+        assert same_bits(host(ds, np.float32, m)[r:r + 1], np.float32([s]))
+
+
 # ------------------------------------------------------------------ weights
 @pytest.mark.parametrize("quant", ALL_FORMATS)
 def test_upload_and_dequantize_rows(gpu, quant):
