@@ -2096,8 +2096,39 @@ static jk_status launch_gemm_tol(hipStream_t s, const WeightDev &w, const jk_act
     }
 }
 
+// Whether a launch of 3 or more tokens takes jk_gemm_few.hip's kernel (the formats and layouts it has).
+// Bit-exact: wherever the tiled launch would leave the 128 x 64 tiles, down to where those smaller tiles
+// have waves enough -- 64 x 64 tiles at more than 2.75 per CU (Q8_0: 2.25), 32 x 32 ones at more than
+// 6 per CU for Q5_K and Q6_K, whose unpacking the small tiles repeat more often. Measured (us, 4096
+// columns, new against tiled): Q4_K 14336 rows 8 / 100 / 192 / 256 tokens 16 / 65 / 93 / 110 against
+// 39 / 73 / 99 / 109, 4096 rows 4 / 50 / 512 / 900 tokens 8 / 13 / 64 / 121 against 34 / 38 / 94 /
+// 108; Q8_0 14336 rows 4 / 100 / 160 tokens 16 / 53 / 78 against 31 / 57 / 72; Q5_K 14336 rows 40 /
+// 128 tokens 33 / 90 against 59 / 86; Q6_K 14336 rows 40 / 100 tokens 56 / 92 against 66 / 89,
+// 4096 x 14336 at 4 / 512 / 768 tokens 26 / 334 / 496 against 201 / 437 / 445.
+// Tolerance mode: up to four 16 x 16 tiles per CU, where splitting K over four waves of a workgroup
+// repeats its loads and unpacking for tokens that are not there (Q4_K 14336 rows 8 tokens 14 against
+// 22, 4096 rows 50 tokens 11 against 19; Q6_K 4096 x 14336 64 tokens 46 against 78); 33 to 48 tokens
+// of the 32-element-group formats, which that kernel pads to 64 (14336 rows 27 against 30); and
+// where the tolerance launch would run the bit-exact tiles (4096 rows 600 tokens 71 against 96).
+static bool few_better(const WeightDev &w, const jk_act_q8 &a, long rows, bool tol) {
+    if (!gemm_few_ok(w, a)) return false;
+    const long ncu = cu_count(), m = (long)a.m;
+    auto tiles = [&](long t) { return (rows + t - 1) / t * ((m + t - 1) / t); };
+    const int tile = gemm_tile(w.quant, rows, m);
+    if (tol && w.cols % 128 == 0) {
+        if (tiles(16) <= 4 * ncu || (m > 32 && m <= 48 && w.quant != JK_Q6_K)) return true;
+        if (tile != 1 || w.quant == JK_Q6_K || 2 * tiles(128) >= 3 * ncu) return false;
+    }
+    switch (tile) {
+    case 0: return false;
+    case 1: return 4 * tiles(64) <= (w.quant == JK_Q8_0 ? 9 : 11) * ncu;
+    default: return w.quant == JK_Q4_K || w.quant == JK_Q4_0 || w.quant == JK_Q8_0 || tiles(32) <= 6 * ncu;
+    }
+}
+
 jk_status launch_gemm_repacked_tol(hipStream_t s, const WeightDev &w, const jk_act_q8 &a, float *y, int r0, int r1) {
     if (a.m <= 2) return launch_gemv_repacked(s, w, a, y, r0, r1);
+    if (few_better(w, a, r1 - r0, true)) return launch_gemm_few(s, w, a, y, r0, r1, cu_count(), true);
     switch (w.quant) {
     case JK_Q8_0: return launch_gemm_tol<JK_Q8_0>(s, w, a, y, r0, r1);
     case JK_Q4_0: return launch_gemm_tol<JK_Q4_0>(s, w, a, y, r0, r1);
@@ -2171,6 +2202,7 @@ jk_status launch_bitlinear_mfma_tol(hipStream_t s, const WeightDev &w, const int
 
 jk_status launch_gemm_repacked(hipStream_t s, const WeightDev &w, const jk_act_q8 &a, float *y, int r0, int r1) {
     if (a.m <= 2) return launch_gemv_repacked(s, w, a, y, r0, r1);
+    if (few_better(w, a, r1 - r0, false)) return launch_gemm_few(s, w, a, y, r0, r1, cu_count(), false);
     switch (w.quant) {
     case JK_Q8_0: return launch_gemm<JK_Q8_0, 1>(s, w, a, y, r0, r1);
     case JK_Q4_0: return launch_gemm<JK_Q4_0, 1>(s, w, a, y, r0, r1);

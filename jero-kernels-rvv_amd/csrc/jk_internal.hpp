@@ -256,6 +256,11 @@ jk_status launch_bitlinear(hipStream_t s, const WeightDev &w, const int8_t *act,
                            const float *act_scales, int m, float *y);
 jk_status launch_gemm_repacked(hipStream_t s, const WeightDev &w, const jk_act_q8 &a, float *y,
                                int r0, int r1);
+// The repacked GEMM for launches with few output tiles (jk_gemm_few.hip): the weights and activations
+// it takes, and the launch (bit-identical to the tiled kernels).
+bool gemm_few_ok(const WeightDev &w, const jk_act_q8 &a);
+jk_status launch_gemm_few(hipStream_t s, const WeightDev &w, const jk_act_q8 &a, float *y, int r0, int r1, long ncu,
+                          bool tol);
 // The same products with each scale group's exact i32 partial (int8 MFMA) rescaled by one fused
 // multiply-add instead of the reference's separately rounded product and sum; outputs within 1e-5
 // of their token's output-row L2 norm. Launches whose bit-exact tiles measured faster run those.

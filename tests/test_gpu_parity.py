@@ -808,6 +808,69 @@ def test_gemm_q8_0_exact_staged_tiles(gpu):
     w.free()
 
 
+FEW_SHAPES = [(3, 37, 512), (16, 100, 2816), (4, 1003, 768), (5, 4201, 512), (33, 4200, 768), (40, 8205, 512),
+              (47, 14000, 512), (61, 12003, 768), (77, 8500, 512)]
+
+
+@pytest.mark.parametrize("quant", [Q8_0, Q4_0, Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("m,rows,cols", FEW_SHAPES + [(3, 70, 64), (9, 70, 448), (21, 4200, 1088)])
+def test_gemm_few_tiles(gpu, quant, m, rows, cols):
+    """The few-tile GEMM on each of its launch shapes (by 16 x 16 output tiles per CU: one, two and four
+    row or token tiles with eight, four and two K waves, and unsplit K): fewer units of 256 elements than
+    waves, a partial last chunk and (448, 1088, 64 columns) a partial last unit, partial row and token
+    tiles, weights with special scales, NaN and Inf activations; equal to the oracle bit for bit on row
+    windows, row slices equal to the full call, and the tolerance mode within its bar (1e-5 of each
+    token's output-row L2 norm, the bar of every tolerance mode)."""
+    torch = gpu
+    if cols % jk.BLOCK_ELEMENTS[quant]:
+        pytest.skip("shape not block aligned")
+    raw = synth.random_weights(quant, rows, cols, seed=m + 7 * quant, specials=True)
+    rng = np.random.default_rng(m + rows)
+    x = rng.standard_normal((m, cols)).astype(np.float32)
+    x[rng.random((m, cols)) < 0.002] = np.nan
+    x[m // 2, cols // 3] = np.inf
+    w = jk.Weight(jk.TensorView("w", quant, [rows, cols], raw), rows, cols)
+    storage, act = gpu_act(torch, x, m, cols)
+    assert jk.gemm_plan(w, act, 0, rows, False) == "gemm_few_kernel"
+    got = gpu_gemm(torch, w, x, m)
+    oact = O.ActQ8(x, m, cols)
+    for r0, r1 in ((0, 33), (rows // 2, rows // 2 + 20), (rows - 35, rows)):
+        r0, r1 = max(r0, 0), min(r1, rows)
+        ref = O.gemm_repacked(quant, [rows, cols], raw, rows, cols, oact, r0, r1)
+        assert same_bits(got[:, r0:r1], ref), (r0, mismatch(got[:, r0:r1], ref))
+    assert same_bits(gpu_gemm(torch, w, x, m, 3, rows - 5), got[:, 3:rows - 5])
+    assert_within_row_norm(gpu_gemm_tol(torch, w, x, m), got)
+    w.free()
+
+
+@pytest.mark.parametrize("quant", [Q8_0, Q4_0, Q4_K, Q5_K, Q6_K])
+def test_gemm_few_tiles_replay(gpu, quant):
+    """The hand-over of running sums between the K waves starts afresh on every launch: repeated calls and
+    graph replays of the few-tile GEMM give the first call's bits."""
+    torch = gpu
+    rows, cols, m = 300, 2816, 7
+    raw = synth.random_weights(quant, rows, cols, seed=quant)
+    x = synth.activations((m, cols), 3)
+    w = jk.Weight(jk.TensorView("w", quant, [rows, cols], raw), rows, cols)
+    storage, act = gpu_act(torch, x, m, cols)
+    y = torch.zeros(m * rows, dtype=torch.float32, device="cuda")
+    jk.dev_gemm_repacked(w, act, y, m * rows, 0, rows)
+    torch.cuda.synchronize()
+    first = y.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        jk.dev_gemm_repacked(w, act, y, m * rows, 0, rows, torch.cuda.current_stream().cuda_stream)
+    for _ in range(5):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int32), first.view(torch.int32))
+        jk.dev_gemm_repacked(w, act, y, m * rows, 0, rows)
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int32), first.view(torch.int32))
+    w.free()
+
+
 TOL128_FORMATS = [Q8_0, Q4_0, Q5_0, Q4_1, Q5_1, IQ4_NL, Q4_K, Q5_K, TQ2_0, I2_S]
 
 
