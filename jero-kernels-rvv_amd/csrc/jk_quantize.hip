@@ -3,6 +3,8 @@
 // Maxima are order-independent, so they are reduced across lanes; sums that the
 // reference accumulates in f32 are accumulated sequentially in one lane in the
 // reference's order; integer sums are reduced across lanes.
+#include <type_traits>
+
 #include "jk_device.hpp"
 
 namespace jk {
@@ -211,43 +213,169 @@ jk_status launch_quantize_act_q8_gated(hipStream_t s, int act, const float *x, c
 // recipe without the RMSNorm step (x_norm = x). One workgroup per row.
 //
 // With the norm, the sum of squares is the reference's sequential f32 sum
-// (dot_product_f32_scalar, lib.rs:770-778), so the row's k dependent additions bound the launch.
-// The products are independent of the order: all threads square the row into LDS a chunk at a
-// time (the next chunk while the first wave adds the current one), and the first wave adds them
-// in order from 16-byte broadcast reads requested 32 values ahead, so an addition waits only for
-// the one before it. (One thread reading and adding straight from global memory waited for a
-// load every few additions: a BitNet feed-forward block of one token, with rows of 2560 and 6912,
-// took 405 us against 59 us now; two 6912 x 2560 products of 128 tokens behind it 137 against 32 us.)
-constexpr int kAbsThreads = 512;
-constexpr int kSqChunk = 2048;  // squares per LDS buffer, a multiple of 32
+// (dot_product_f32_scalar, lib.rs:770-778): k additions that each wait for the one before, about 9
+// cycles each (26 us for 6912). It is put together in parallel instead, bit for bit: while the
+// running sum stays inside one binade it is an integer A times its ulp u, and adding x >= 0 gives
+// RNE(A + x / u) u, so A grows by round(x / u) whatever A is -- except where x / u lies exactly
+// between two integers (a tie goes to the even neighbour, which depends on A) or the sum leaves the
+// binade. An approximate prefix sum tells each element's binade; the increments are added by an
+// integer scan; and the elements where the rule does not hold (within 2e-5 of a power of two, about
+// one per doubling of the sum; ties; the first element; NaN and Inf; sums near the ends of the
+// exponent range) are added one by one by the first wave, between them the scan's increments as one
+// integer addition to the float's bits. That addition is checked to start and to end in the
+// expected binade; if it does not, or if there are too many such elements, the first wave adds the
+// whole row one by one. Normal rows of 2560 and 6912 have 21 and 23 such elements: 7.8 and 10.5 us a
+// launch, against 12.7 and 29.3 us with every element added from LDS by the first wave (about 190 us
+// by one thread from global memory). What bounds it now: the three scans' cross-lane steps, the
+// elements added one by one (a scalar round trip each) and three passes over the row.
+constexpr int kAbsThreads = 1024;
+constexpr int kSqMax = 14336;     // squares held in LDS at once (14 per thread); longer rows go in such pieces
+constexpr int kSqSerial = 256;    // pieces up to this length are added one by one
+constexpr int kSqEvents = 256;    // elements added one by one otherwise, at most
 
-// acc + s[0] + s[1] + ... + s[n - 1], in order (s: 16-byte aligned LDS, the same for every lane)
+struct SumLds {
+    float part[kAbsThreads / 64];                    // per wave: sum of its squares
+    int inc[kAbsThreads / 64], cnt[kAbsThreads / 64];  // increments and events
+    int4 ev[kSqEvents];                              // position, increments before it, binade, the square's bits
+    int tail_eb;                                     // binade after the last element
+};
+
+// acc + s[0] + s[1] + ... + s[n - 1], in order (s: LDS, the same for every lane; n >= 1). Reads are
+// requested sixteen ahead and unconditional (past the end the last value, replaced by -0.0, the
+// identity of f32 addition): a read behind a test waits for itself.
 __device__ __forceinline__ float ordered_sum(float acc, const float *s, int n) {
-    const float4 *s4 = reinterpret_cast<const float4 *>(s);
-    const int n32 = n / 32;
-    float4 cur[8], nxt[8];
+    constexpr int N = 16;
+    float cur[N], nxt[N];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) cur[i] = s4[i];  // (the buffer holds at least 32 values)
-    for (int c = 0; c < n32; ++c) {
-        const int cn = min(c + 1, n32 - 1);
+    for (int i = 0; i < N; ++i) cur[i] = s[min(i, n - 1)];
+    for (int c = 0; c < n; c += N) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) nxt[i] = s4[8 * cn + i];
+        for (int i = 0; i < N; ++i) nxt[i] = s[min(c + N + i, n - 1)];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc = (((acc + cur[i].x) + cur[i].y) + cur[i].z) + cur[i].w;
+        for (int i = 0; i < N; ++i) cur[i] = c + i < n ? cur[i] : -0.0f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) cur[i] = nxt[i];
+        for (int i = 0; i < N; ++i) acc += cur[i];
+#pragma unroll
+        for (int i = 0; i < N; ++i) cur[i] = nxt[i];
     }
-    for (int i = 32 * n32; i < n; ++i) acc += s[i];
     return acc;
 }
 
+// The same sum of n values >= 0 (or NaN) by the whole workgroup, as described above; the result is
+// the first wave's. PER: values per thread, odd (the threads' reads then fall on distinct banks).
+template <int PER>
+__device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *sq, int n, SumLds &L) {
+    constexpr int NW = kAbsThreads / 64;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int lo = t * PER;
+    float v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) v[i] = sq[min(lo + i, n - 1)];
+    float part = 0.0f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        v[i] = lo + i < n ? v[i] : 0.0f;
+        part += v[i];
+    }
+    float incl = part;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const float u = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += u;
+    }
+    if (lane == 63) L.part[wave] = incl;
+    __syncthreads();
+    float pre = acc0 + (incl - part);  // approximate sum before the thread's first element
+#pragma unroll
+    for (int i = 0; i < NW; ++i) pre += i < wave ? L.part[i] : 0.0f;
+    // element i after an approximate sum p: its binade, whether it goes by the rule, and its increment
+    auto element = [&](int i, float p, uint32_t &eb, bool &ok) {
+        eb = __float_as_uint(p * 0.99998f) >> 23;
+        const uint32_t ee = __float_as_uint((p + v[i]) * 1.00002f) >> 23;
+        const float to_ulp = __uint_as_float((277u - min(max(eb, 30u), 220u)) << 23);  // 1 / u, a power of two
+        const float w = v[i] * to_ulp, fl = floorf(w), fr = w - fl;
+        ok = eb == ee && eb >= 30 && eb <= 220 && w < 16777216.0f && fr != 0.5f;
+        return ok ? (int)fl + (fr > 0.5f ? 1 : 0) : 0;
+    };
+    uint32_t events = 0;
+    int inc = 0;
+    float p = pre;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        uint32_t eb;
+        bool ok;
+        const int r = element(i, p, eb, ok);
+        p += v[i];
+        const bool live = lo + i < n;
+        inc += live ? r : 0;
+        events |= (uint32_t)(live && !ok) << i;
+        if (lo + i == n - 1) L.tail_eb = (int)eb;
+    }
+    int pi = inc, pc = __popc(events);
+    const int cnt = pc;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int ui = __shfl_up(pi, o, 64), uc = __shfl_up(pc, o, 64);
+        if (lane >= o) pi += ui, pc += uc;
+    }
+    if (lane == 63) L.inc[wave] = pi, L.cnt[wave] = pc;
+    __syncthreads();
+    int ri = pi - inc, ci = pc - cnt, total_i = 0, total_c = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        ri += i < wave ? L.inc[i] : 0, ci += i < wave ? L.cnt[i] : 0;
+        total_i += L.inc[i], total_c += L.cnt[i];
+    }
+    if (events) {
+        p = pre;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            uint32_t eb;
+            bool ok;
+            const int r = element(i, p, eb, ok);
+            p += v[i];
+            if ((events >> i) & 1u) {
+                if (ci < kSqEvents) L.ev[ci] = make_int4(lo + i, ri, (int)eb, __float_as_int(v[i]));
+                ++ci;
+            }
+            ri += r;
+        }
+    }
+    __syncthreads();
+    if (t >= 64) return 0.0f;
+    uint32_t bits = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(acc0));
+    bool fits = total_c <= kSqEvents;
+    int pos = -1, done = 0;  // the last element added, and the increments added (scalars)
+    // the increments up to (not including) element p, all in binade e
+    auto advance = [&](int p, int upto, uint32_t e) {
+        const uint32_t to = bits + (uint32_t)(upto - done);
+        if (p > pos + 1 && ((bits >> 23) != e || (to >> 23) != e)) fits = false;
+        bits = to, done = upto;
+    };
+    for (int g = 0; fits && g < total_c; g += 64) {
+        const int4 ev = L.ev[min(g + lane, total_c - 1)];  // lane l: event g + l
+        for (int j = 0; j < min(64, total_c - g); ++j) {
+            const int p = __builtin_amdgcn_readlane(ev.x, j);
+            advance(p, __builtin_amdgcn_readlane(ev.y, j), (uint32_t)__builtin_amdgcn_readlane(ev.z, j));
+            const float acc = __uint_as_float(bits) + __int_as_float(__builtin_amdgcn_readlane(ev.w, j));
+            bits = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(acc));
+            pos = p;
+        }
+    }
+    advance(n, total_i, (uint32_t)__builtin_amdgcn_readfirstlane(L.tail_eb));
+    return fits ? __uint_as_float(bits) : ordered_sum(acc0, sq, n);
+}
+
 // V4: k % 4 == 0 and 16-byte aligned rows and norm weights (the codes are then stored 4 at a time)
-template <bool V4>
+// PER: squares per thread of a piece (odd, see parallel_ordered_sum); a row longer than PER values per
+// thread is summed in pieces of 14 per thread
+template <bool V4, int PER>
 __global__ __launch_bounds__(kAbsThreads) void absmax_i8_kernel(const float *__restrict__ x,
                                                                 const float *__restrict__ nw, size_t k, float eps,
                                                                 int8_t *__restrict__ q, float *__restrict__ scales) {
     constexpr int NT = kAbsThreads, VE = V4 ? 4 : 1;
-    __shared__ __align__(16) float s_sq[2][kSqChunk];
+    __shared__ __align__(16) float s_sq[kSqMax];
+    __shared__ __align__(16) SumLds s_sum;
     __shared__ float s_inv;
     __shared__ float s_max[NT / 64];
     const size_t row = blockIdx.x;
@@ -255,26 +383,26 @@ __global__ __launch_bounds__(kAbsThreads) void absmax_i8_kernel(const float *__r
     const int t = threadIdx.x;
     float inv = 1.0f;
     if (nw) {
-        auto fill = [&](size_t c0, float *dst, int first, int n) {  // threads first .. first + n - 1
-            const int len = (int)min((size_t)kSqChunk, k - c0);
-            for (int i = VE * (t - first); i < len; i += VE * n) {
+        float sum_sq = 0.0f;  // (the first wave's)
+        for (size_t c0 = 0; c0 < k; c0 += kSqMax) {
+            const int len = (int)min((size_t)kSqMax, k - c0);
+            if (c0 > 0) {
+                if (t == 0) s_inv = sum_sq;
+                __syncthreads();  // the piece before is summed; its running sum is every thread's
+                sum_sq = s_inv;
+            }
+            for (int i = VE * t; i < len; i += VE * NT) {
                 if constexpr (V4) {
                     const float4 v = *reinterpret_cast<const float4 *>(src + c0 + i);
-                    *reinterpret_cast<float4 *>(dst + i) = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
+                    *reinterpret_cast<float4 *>(s_sq + i) = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
                 } else {
                     const float v = src[c0 + i];
-                    dst[i] = v * v;
+                    s_sq[i] = v * v;
                 }
             }
-        };
-        fill(0, s_sq[0], 0, NT);
-        __syncthreads();
-        float sum_sq = 0.0f;
-        int buf = 0;
-        for (size_t c0 = 0; c0 < k; c0 += kSqChunk, buf ^= 1) {
-            if (t < 64) sum_sq = ordered_sum(sum_sq, s_sq[buf], (int)min((size_t)kSqChunk, k - c0));
-            else if (c0 + kSqChunk < k) fill(c0 + kSqChunk, s_sq[buf ^ 1], 64, NT - 64);
             __syncthreads();
+            if (len <= kSqSerial) sum_sq = t < 64 ? ordered_sum(sum_sq, s_sq, len) : 0.0f;
+            else sum_sq = parallel_ordered_sum<PER>(sum_sq, s_sq, len, s_sum);
         }
         if (t == 0) {
             const float mean_sq = sum_sq / (float)k;
@@ -332,9 +460,15 @@ __global__ __launch_bounds__(kAbsThreads) void absmax_i8_kernel(const float *__r
 jk_status launch_absmax_i8(hipStream_t s, const float *x, const float *norm_w, size_t m, size_t k, float eps,
                            int8_t *q, float *scales) {
     const bool v4 = k % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)norm_w % 16 == 0 && (uintptr_t)q % 4 == 0;
-    const dim3 grid((unsigned)m), block(kAbsThreads);
-    if (v4) hipLaunchKernelGGL(absmax_i8_kernel<true>, grid, block, 0, s, x, norm_w, k, eps, q, scales);
-    else hipLaunchKernelGGL(absmax_i8_kernel<false>, grid, block, 0, s, x, norm_w, k, eps, q, scales);
+    auto launch = [&](auto per) {
+        constexpr int PER = decltype(per)::value;
+        const dim3 grid((unsigned)m), block(kAbsThreads);
+        if (v4) hipLaunchKernelGGL((absmax_i8_kernel<true, PER>), grid, block, 0, s, x, norm_w, k, eps, q, scales);
+        else hipLaunchKernelGGL((absmax_i8_kernel<false, PER>), grid, block, 0, s, x, norm_w, k, eps, q, scales);
+    };
+    if (k <= 3 * kAbsThreads) launch(std::integral_constant<int, 3>());
+    else if (k <= 7 * kAbsThreads) launch(std::integral_constant<int, 7>());
+    else launch(std::integral_constant<int, 15>());
     return check_launch("absmax_i8_kernel");
 }
 

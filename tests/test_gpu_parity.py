@@ -164,15 +164,20 @@ def test_absmax_quantizers(gpu, k):
 
 
 @pytest.mark.parametrize("offset", [0, 1])
-@pytest.mark.parametrize("k", [1, 3, 31, 32, 33, 2047, 2048, 2049, 4100, 6911])
+@pytest.mark.parametrize("k", [1, 3, 7, 16, 33, 255, 256, 257, 1023, 1025, 2560, 4100, 6911, 14336, 14337, 29000])
 def test_subln_absmax_sizes(gpu, k, offset):
-    """The ordered sum of squares around its 32-value reads and 2048-value LDS buffers, and rows that
-    are not 16-byte aligned; an Inf and a NaN row."""
+    """The ordered sum of squares: added one by one up to 256 values, in parallel beyond, in pieces of
+    14336; aligned rows and rows that are not. Row kinds: normal values of mixed magnitude, Inf, NaN,
+    ties everywhere (multiples of 1/4), equal powers of two, mostly zeros, growing by 40 binades, tiny
+    and huge values, all zero."""
     torch = gpu
     rng = np.random.default_rng(k + offset)
-    m = 3
-    x = (rng.standard_normal((m, k)) * rng.choice([1e-3, 1, 50], (m, k))).astype(np.float32)
+    z = rng.standard_normal((10, k))
+    x = np.stack([z[0] * rng.choice([1e-3, 1, 50], k), z[1], z[2], np.round(z[3] * 4) / 4, np.full(k, 0.25),
+                  np.where(rng.random(k) < 0.95, 0, z[5]), z[6] * np.exp2(np.linspace(-20, 20, k)), z[7] * 1e-18,
+                  z[8] * 1e17, z[9] * 0]).astype(np.float32)
     x[1, k // 2], x[2, 0] = np.inf, np.nan
+    m = len(x)
     w = rng.uniform(-1.5, 1.5, k).astype(np.float32)
     dx = torch.zeros(m * k + 4, dtype=torch.float32, device="cuda")
     dx[offset:offset + m * k] = torch.from_numpy(x.reshape(-1)).cuda()
@@ -184,8 +189,8 @@ def test_subln_absmax_sizes(gpu, k, offset):
     got = host(dq, np.int8, m * k + 4)[offset:offset + m * k].reshape(m, k)
     for r in range(m):
         q, s = O.subln_quantize_absmax_i8(x[r], w, 1e-5)
-        assert np.array_equal(got[r], q)
-        assert same_bits(host(ds, np.float32, m)[r:r + 1], np.float32([s]))
+        assert np.array_equal(got[r], q), r
+        assert same_bits(host(ds, np.float32, m)[r:r + 1], np.float32([s])), r
 
 
 # ------------------------------------------------------------------ weights
