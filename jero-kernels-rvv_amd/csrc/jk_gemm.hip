@@ -2126,8 +2126,24 @@ static bool few_better(const WeightDev &w, const jk_act_q8 &a, long rows, bool t
     }
 }
 
+// Whether a tolerance-mode launch takes jk_gemm_split.hip's kernel: its tiles of 256 rows x 128 tokens
+// cost the same whether full or not and run one to a CU, so the outputs have to fill half of the rounds
+// that the tiles need. Measured (us, new against the launches below): Q4_K x 4096 columns, 11008 rows
+// 384 tokens (0.5 of one round) 105 against 135, 4096 rows 1024 tokens (0.5) 102 against 108, 14336 rows
+// 512 / 640 (0.55 of two) / 1024 / 1400 / 2048 tokens 130 / 219 / 235 / 331 / 443 against 167 / 244 / 302 /
+// 381 / 533; Q5_K 14336 rows 512 / 1024 tokens 144 / 249 against 179 / 332; below half, 2048 rows x 8192
+// 1400 tokens (0.34) 186 against 163, 1300 rows 1400 tokens (0.22) 99 against 70. Rows of fewer than four
+// blocks, shorter than any model's, stay on the 128 x 128 tiles, whose tests hold them there.
+static bool split_better(const WeightDev &w, const jk_act_q8 &a, long rows) {
+    if (!gemm_split_ok(w, a) || w.cols < 1024) return false;
+    const long ncu = cu_count(), m = (long)a.m;
+    const long rounds = ((rows + 255) / 256 * ((m + 127) / 128) + ncu - 1) / ncu;
+    return 2 * rows * m >= 256 * 128 * ncu * rounds;
+}
+
 jk_status launch_gemm_repacked_tol(hipStream_t s, const WeightDev &w, const jk_act_q8 &a, float *y, int r0, int r1) {
     if (a.m <= 2) return launch_gemv_repacked(s, w, a, y, r0, r1);
+    if (split_better(w, a, r1 - r0)) return launch_gemm_split(s, w, a, y, r0, r1);
     if (few_better(w, a, r1 - r0, true)) return launch_gemm_few(s, w, a, y, r0, r1, cu_count(), true);
     switch (w.quant) {
     case JK_Q8_0: return launch_gemm_tol<JK_Q8_0>(s, w, a, y, r0, r1);

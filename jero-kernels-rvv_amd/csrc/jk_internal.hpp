@@ -261,6 +261,9 @@ jk_status launch_gemm_repacked(hipStream_t s, const WeightDev &w, const jk_act_q
 bool gemm_few_ok(const WeightDev &w, const jk_act_q8 &a);
 jk_status launch_gemm_few(hipStream_t s, const WeightDev &w, const jk_act_q8 &a, float *y, int r0, int r1, long ncu,
                           bool tol);
+// The tolerance-mode GEMM of Q4_K and Q5_K with the group scales in f16 operands (jk_gemm_split.hip).
+bool gemm_split_ok(const WeightDev &w, const jk_act_q8 &a);
+jk_status launch_gemm_split(hipStream_t s, const WeightDev &w, const jk_act_q8 &a, float *y, int r0, int r1);
 // The same products with each scale group's exact i32 partial (int8 MFMA) rescaled by one fused
 // multiply-add instead of the reference's separately rounded product and sum; outputs within 1e-5
 // of their token's output-row L2 norm. Launches whose bit-exact tiles measured faster run those.

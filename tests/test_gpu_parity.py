@@ -876,6 +876,35 @@ def test_gemm_few_tiles_replay(gpu, quant):
     w.free()
 
 
+@pytest.mark.parametrize("quant", [Q4_K, Q5_K])
+@pytest.mark.parametrize("m,rows,cols", [(500, 8403, 1024), (2049, 2064, 1280), (300, 14343, 1792)])
+def test_gemm_split(gpu, quant, m, rows, cols):
+    """Tolerance-mode GEMM with the group scales in f16 operands: partial last row and token tiles, rows
+    that are and are not whole 16-byte stores, even and odd block counts, weights with special scales,
+    NaN and Inf activations in some tokens, the largest quants, scales and mins with an activation row of
+    equal values (the largest group sums), and one of tiny values. Within 1e-5 of each token's output-row
+    L2 norm of the bit-exact GEMM (the bar of every tolerance mode), NaN where that is, a row slice
+    equal to the full call."""
+    torch = gpu
+    raw = synth.random_weights(quant, rows, cols, seed=m + quant, specials=True)
+    blk = np.asarray(raw).view(np.uint8).reshape(rows, cols // 256, jk.BLOCK_BYTES[quant])
+    blk[5:9, :, 4:] = 0xFF
+    rng = np.random.default_rng(m + rows)
+    x = rng.standard_normal((m, cols)).astype(np.float32)
+    x[3], x[4] = 1.0, x[4] * np.float32(1e-20)
+    x[7, cols // 3], x[m - 2, 5], x[11, 40] = np.inf, -np.inf, np.nan
+    w = jk.Weight(jk.TensorView("w", quant, [rows, cols], raw), rows, cols)
+    exact = gpu_gemm(torch, w, x, m)
+    tol = gpu_gemm_tol(torch, w, x, m, expect="gemm_split_kernel")
+    assert np.array_equal(np.isnan(tol), np.isnan(exact))
+    fin = ~np.isnan(exact).any(axis=1)
+    assert fin.sum() >= m - 3
+    worst = assert_within_row_norm(tol[fin], exact[fin])
+    assert same_bits(gpu_gemm_tol(torch, w, x, m, 5, rows - 2, expect="gemm_split_kernel"), tol[:, 5:rows - 2])
+    print(f"gemm split {quant} {rows}x{cols} M={m}: worst error / row norm {worst:.2e}")
+    w.free()
+
+
 TOL128_FORMATS = [Q8_0, Q4_0, Q5_0, Q4_1, Q5_1, IQ4_NL, Q4_K, Q5_K, TQ2_0, I2_S]
 
 
