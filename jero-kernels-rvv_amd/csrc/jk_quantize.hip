@@ -223,8 +223,10 @@ jk_status launch_quantize_act_q8_gated(hipStream_t s, int act, const float *x, c
 // one per doubling of the sum; ties; the first element; NaN and Inf; sums near the ends of the
 // exponent range) are added one by one by the first wave, between them the scan's increments as one
 // integer addition to the float's bits. That addition is checked to start and to end in the
-// expected binade; if it does not, or if there are too many such elements, the first wave adds the
-// whole row one by one. Normal rows of 2560 and 6912 have 21 and 23 such elements: 7.8 and 10.5 us a
+// expected binade, and all its elements to have been given that binade (a thread's approximate prefix
+// can lie a few ulps below the end of the thread before it, put together in another order, and fall
+// back into the binade below); where a check fails, or with too many such elements, the first wave adds
+// the whole row one by one. Normal rows of 2560 and 6912 have 21 and 23 such elements: 7.8 and 10.5 us a
 // launch, against 12.7 and 29.3 us with every element added from LDS by the first wave (about 190 us
 // by one thread from global memory). What bounds it now: the three scans' cross-lane steps, the
 // elements added one by one (a scalar round trip each) and three passes over the row.
@@ -237,6 +239,8 @@ struct SumLds {
     float part[kAbsThreads / 64];                    // per wave: sum of its squares
     int inc[kAbsThreads / 64], cnt[kAbsThreads / 64];  // increments and events
     int4 ev[kSqEvents];                              // position, increments before it, binade, the square's bits
+    uint32_t first[kAbsThreads / 64], last[kAbsThreads / 64];  // binades of the wave's first and last elements
+    int split[kAbsThreads / 64];                     // whether a run changes its binade between two threads of the wave
     int tail_eb;                                     // binade after the last element
 };
 
@@ -300,6 +304,8 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
     uint32_t events = 0;
     int inc = 0;
     float p = pre;
+    uint32_t first = 0, last = 0;  // binades of the first and the last element (kNoRun: no run goes on past it)
+    constexpr uint32_t kNoRun = 1u << 16;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         uint32_t eb;
@@ -310,7 +316,16 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
         inc += live ? r : 0;
         events |= (uint32_t)(live && !ok) << i;
         if (lo + i == n - 1) L.tail_eb = (int)eb;
+        if (i == 0) first = live ? eb : kNoRun;
+        if (i == PER - 1) last = live && ok ? eb : kNoRun;
     }
+    // the elements of a run share a binade: within a thread by construction (an element by the rule ends in
+    // the binade that the next one starts from), from one thread to the next by this test
+    const uint32_t before = __shfl_up(last, 1, 64);
+    const bool split = lane > 0 && ((before | first) & kNoRun) == 0 && before != first;
+    const uint64_t any_split = __ballot(split);
+    if (lane == 0) L.first[wave] = first, L.split[wave] = any_split != 0;
+    if (lane == 63) L.last[wave] = last;
     int pi = inc, pc = __popc(events);
     const int cnt = pc;
 #pragma unroll
@@ -345,6 +360,10 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
     if (t >= 64) return 0.0f;
     uint32_t bits = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(acc0));
     bool fits = total_c <= kSqEvents;
+    for (int i = 0; i < NW; ++i) {
+        fits = fits && !L.split[i];
+        if (i > 0) fits = fits && (((L.last[i - 1] | L.first[i]) & kNoRun) != 0 || L.last[i - 1] == L.first[i]);
+    }
     int pos = -1, done = 0;  // the last element added, and the increments added (scalars)
     // the increments up to (not including) element p, all in binade e
     auto advance = [&](int p, int upto, uint32_t e) {

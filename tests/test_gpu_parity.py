@@ -193,6 +193,32 @@ def test_subln_absmax_sizes(gpu, k, offset):
         assert same_bits(host(ds, np.float32, m)[r:r + 1], np.float32([s])), r
 
 
+@pytest.mark.parametrize("k,per", [(2800, 3), (4859, 7), (7381, 15)])
+def test_subln_absmax_lagging_sum(gpu, k, per):
+    """Rows whose ordered sum lags the plain prefix sums from which the parallel form takes each element's
+    binade: after a first value near 0.56, thousands of squares of less than half an ulp are rounded away one
+    by one; one value carries the prefix to 1 / 0.99998, where elements start to count as past 1, while the
+    ordered sum is below 1; squares of 1.5 to 1.75 ulp follow to the end of a thread's `per` elements, and one
+    more. There the next thread's prefix may lie back below that line."""
+    torch = gpu
+    rng = np.random.default_rng(k)
+    m, ulp, at = 300, 2.0 ** -24, k - 1 - per
+    sq = np.empty((m, k))
+    sq[:] = rng.uniform(0.3, 0.48, (m, 1)) * ulp
+    sq[:, 0] = rng.uniform(0.7, 0.8, m) ** 2
+    sq[:, at + 1:] = rng.uniform(1.5, 1.75, (m, 1)) * ulp
+    sq[:, at] = 1 / 0.99998 + rng.uniform(-4, 4, m) * ulp - sq[:, :at].sum(1) - (per - 1) * sq[:, -1]
+    x = np.sqrt(sq).astype(np.float32)
+    w = np.ones(k, np.float32)
+    dq, ds = empty(torch, m * k), empty(torch, 4 * m)
+    jk.dev_subln_quantize_absmax_i8(dev(torch, x), dev(torch, w), m, k, 1e-5, dq, ds)
+    torch.cuda.synchronize()
+    ref = [O.subln_quantize_absmax_i8(r, w, 1e-5) for r in x]
+    scales = np.float32([s for _, s in ref])
+    assert same_bits(host(ds, np.float32, m), scales), mismatch(host(ds, np.float32, m), scales)
+    assert np.array_equal(host(dq, np.int8, m * k).reshape(m, k), np.stack([q for q, _ in ref]))
+
+
 # ------------------------------------------------------------------ weights
 @pytest.mark.parametrize("quant", ALL_FORMATS)
 def test_upload_and_dequantize_rows(gpu, quant):
