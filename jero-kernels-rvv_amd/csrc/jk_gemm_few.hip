@@ -339,11 +339,11 @@ __global__ __launch_bounds__(64 * RW * TW * KW) void gemm_few_kernel(WeightDev w
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int jl = lane & 15, kq = lane >> 4;
     const int kw = wave / (RW * TW), tile = wave % (RW * TW), rw = tile % RW, tw = tile / RW;
-    // a row tile's token tiles on one XCD (workgroup i runs on XCD i % 8)
+    // an eighth of the tiles per XCD (workgroup i runs on XCD i % 8), a row tile's token tiles together
     const int ntn = (r1 - r0 + 16 * RW - 1) / (16 * RW), ntm = ((int)a.m + 16 * TW - 1) / (16 * TW);
-    const int wg = (int)blockIdx.x, local = wg >> 3;
-    const int tn = (local / ntm) * 8 + (wg & 7), tm = local % ntm;
-    if (tn >= ntn) return;  // workgroup-uniform
+    const int wg = (int)blockIdx.x, t = (wg & 7) * ((int)gridDim.x >> 3) + (wg >> 3);
+    if (t >= ntn * ntm) return;  // workgroup-uniform
+    const int tn = t / ntm, tm = t % ntm;
     const int n0 = r0 + 16 * RW * tn, m0 = 16 * TW * tm, M = (int)a.m;
     const int steps = w.cols / 32, units = (steps + 7) / 8, nchunks = (units + KU - 1) / KU;
     const int row = 16 * rw + jl, tok = 16 * tw + jl;
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(64 * RW * TW * KW) void gemm_few_kernel(WeightDev w
 template <int Q, int RW, int TW, int KU, int KW>
 static jk_status launch_few_t(hipStream_t s, const WeightDev &w, const jk_act_q8 &a, float *y, int r0, int r1, bool tol) {
     const size_t ntn = (size_t)(r1 - r0 + 16 * RW - 1) / (16 * RW), ntm = (a.m + 16 * TW - 1) / (16 * TW);
-    const dim3 grid((unsigned)((ntn + 7) / 8 * 8 * ntm)), block(64 * RW * TW * KW);
+    const dim3 grid((unsigned)((ntn * ntm + 7) / 8 * 8)), block(64 * RW * TW * KW);
     if (tol)
         JK_LAUNCH("gemm_few_kernel<tolerance>", (gemm_few_kernel<Q, RW, TW, KU, KW, true>), grid, block, 0, s, w, a, y, r0, r1);
     else
