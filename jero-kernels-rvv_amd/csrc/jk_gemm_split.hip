@@ -10,6 +10,11 @@
 // and per 256-element block acc = fma(d, part, acc) and the mins, acc = fma(-dmin, sum(xsum * mn), acc),
 // whose sums over the 8 groups are two bf16 MFMAs: xsum as three bf16 numbers (24 bits), mn exact.
 //
+// Formed before d and dmin come in, a block's sums can pass f32's range where the outputs do not: they
+// reach 2^12 times its xs (with the operands' 2^-14) and 2^9 times its xsum. Both are taken times 2^-13,
+// which d and dmin give back, so that no finite xs or xsum overflows; the quantizer's xs are zero or
+// at least 1e-30 / 127, far enough from f32's smallest.
+//
 // A workgroup owns 256 weight rows x 128 tokens, a wave 32 x 128. Weights go from global memory straight
 // into one of two LDS stages a 256-element block ahead, activations through registers a 64-element
 // quarter ahead, converted to f16 once per workgroup; a wave unpacks the weights that it multiplies.
@@ -33,13 +38,14 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
 constexpr int kSplitN = 256, kSplitM = 128, kSplitThreads = 512;
+constexpr float kSplitDown = 0x1p-13f, kSplitUp = 0x1p13f;
 
 template <int Q> struct alignas(16) SplitLds {
     static constexpr int P = fmt_of(Q).chunks;
     uint8_t x[2][kSplitM][128];         // [stage][token]: 8 16-byte pieces of f16, XORed with the token
-    float xs[2][kSplitM][8];            // [block & 1][token][group]
-    uint16_t xm[2][4][kSplitM][8];      // the groups' sums in three bf16 parts, and zeros
-    float d[kSplitN], dm[kSplitN];      // the rows' 2^14 d and dmin
+    float xs[2][kSplitM][8];            // [block & 1][token][group], times 2^-13
+    uint16_t xm[2][4][kSplitM][8];      // the groups' sums times 2^-13 in three bf16 parts, and zeros
+    float d[kSplitN], dm[kSplitN];      // the rows' 2^27 d and 2^13 dmin
     uint8_t w[2][P][kSplitN][16];       // [stage][plane][row] (last: the others within an instruction's offset)
 };
 
@@ -94,14 +100,15 @@ gemm_split_kernel(WeightDev w, jk_act_q8 a, float *__restrict__ y, int r0, int r
     };
     // the token's scales and sums of groups 2 part, 2 part + 1 of block b
     auto sstore = [&](float2 fs, float2 fm, int b) {
-        *reinterpret_cast<float2 *>(&L.xs[b & 1][(tv >> 2)][2 * (tv & 3)]) = fs;
-        float v0 = fm.x, v1 = fm.y;
+        *reinterpret_cast<float2 *>(&L.xs[b & 1][(tv >> 2)][2 * (tv & 3)]) = float2{fs.x * kSplitDown, fs.y * kSplitDown};
+        float v0 = fm.x * kSplitDown, v1 = fm.y * kSplitDown;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {  // (truncated to 8 bits each: the differences are exact)
             const uint32_t c0 = __float_as_uint(v0) & 0xFFFF0000u, c1 = __float_as_uint(v1) & 0xFFFF0000u;
             *reinterpret_cast<uint32_t *>(&L.xm[b & 1][k][(tv >> 2)][2 * (tv & 3)]) = (c0 >> 16) | c1;
-            v0 -= __uint_as_float(c0);
-            v1 -= __uint_as_float(c1);
+            // (nothing is left of an infinite sum, whose difference from itself is NaN)
+            v0 = __builtin_isinf(v0) ? 0.0f : v0 - __uint_as_float(c0);
+            v1 = __builtin_isinf(v1) ? 0.0f : v1 - __uint_as_float(c1);
         }
     };
     // this wave's share of the weight loads: plane wave / 4 + 2 i, 64 rows
@@ -218,8 +225,8 @@ gemm_split_kernel(WeightDev w, jk_act_q8 a, float *__restrict__ y, int r0, int r
             }
             if (j == 1 && wave < kSplitN / 64) {  // (the last block's have been read)
                 const uint32_t dd = *reinterpret_cast<const uint32_t *>(L.w[b & 1][0][tv]);
-                L.d[tv] = 16384.0f * f16_finite(dd & 0xFFFFu);
-                L.dm[tv] = f16_finite(dd >> 16);
+                L.d[tv] = 16384.0f * kSplitUp * f16_finite(dd & 0xFFFFu);
+                L.dm[tv] = kSplitUp * f16_finite(dd >> 16);
             }
             if (j == 2) sstore(fs, fm, b + 1);
             if (j == 0) {

@@ -931,6 +931,33 @@ def test_gemm_split(gpu, quant, m, rows, cols):
     w.free()
 
 
+@pytest.mark.parametrize("quant", [Q4_K, Q5_K])
+def test_gemm_split_range(gpu, quant):
+    """The split GEMM sums a block's groups before d and dmin scale them: activations of up to 1e36 give the
+    finite outputs of the bit-exact GEMM, as do those near the quantizer's zero threshold of 1e-30, and a
+    group whose activation sum overflows gives its infinities and NaN. Per-token scales of 1e-29 to 1e36, all
+    within 1e-5 of each token's output-row L2 norm; block scales near 2e-5, so that the bit-exact terms stay
+    finite too."""
+    torch = gpu
+    m, rows, cols = 300, 14343, 1024
+    raw = synth.gguf_weights(quant, rows, cols, seed=quant)
+    rng = np.random.default_rng(quant)
+    blk = raw.reshape(-1, jk.BLOCK_BYTES[quant])
+    blk[:, :4] = rng.uniform(1e-5, 3e-5, (len(blk), 2)).astype(np.float16).view(np.uint8)
+    x = rng.standard_normal((m, cols)) * np.float64(10.0) ** rng.integers(-29, 37, (m, 1))
+    x[0] *= 1e36 / np.abs(x[0]).max()
+    x[1], x[1, 64:96] = 0, 1.2e37
+    x = x.astype(np.float32)
+    assert np.isfinite(x).all()
+    w = jk.Weight(jk.TensorView("w", quant, [rows, cols], raw), rows, cols)
+    exact = gpu_gemm(torch, w, x, m)
+    tol = gpu_gemm_tol(torch, w, x, m, expect="gemm_split_kernel")
+    assert np.array_equal(np.isnan(tol[1]), np.isnan(exact[1])) and np.array_equal(tol[1] == -np.inf, exact[1] == -np.inf)
+    assert not np.isfinite(exact[1]).any() and np.isfinite(exact[2:]).all()
+    assert_within_row_norm(np.delete(tol, 1, 0), np.delete(exact, 1, 0))
+    w.free()
+
+
 TOL128_FORMATS = [Q8_0, Q4_0, Q5_0, Q4_1, Q5_1, IQ4_NL, Q4_K, Q5_K, TQ2_0, I2_S]
 
 
