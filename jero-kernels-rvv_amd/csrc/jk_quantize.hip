@@ -209,10 +209,73 @@ jk_status launch_quantize_act_q8_gated(hipStream_t s, int act, const float *x, c
     return check_launch("quantize_act_q8_kernel");
 }
 
-// subln_quantize_absmax_i8 (lib.rs:1042-1101) per row; norm_w == nullptr gives the same
-// recipe without the RMSNorm step (x_norm = x). One workgroup per row.
+// quantize_absmax_i8 of a row, with NORM of x * inv * nw: the maximum over the workgroup, then the codes.
+// V4: k % 4 == 0 and 16-byte aligned rows and norm weights (the codes are then stored 4 at a time).
+// NT: threads of the workgroup.
+template <bool V4, bool NORM, int NT>
+__device__ __forceinline__ void absmax_codes(const float *src, const float *nw, float inv, size_t k, int8_t *dst,
+                                             float *scale_out) {
+    constexpr int VE = V4 ? 4 : 1;
+    __shared__ float s_max[NT / 64];
+    const int t = threadIdx.x;
+    auto xnorm = [&](size_t i, float (&o)[VE]) {  // of elements i .. i + VE - 1
+        if constexpr (V4) {
+            const float4 v = *reinterpret_cast<const float4 *>(src + i);
+            o[0] = v.x, o[1] = v.y, o[2] = v.z, o[3] = v.w;
+            if constexpr (NORM) {
+                const float4 g = *reinterpret_cast<const float4 *>(nw + i);
+                o[0] = o[0] * inv * g.x, o[1] = o[1] * inv * g.y, o[2] = o[2] * inv * g.z, o[3] = o[3] * inv * g.w;
+            }
+        } else {
+            o[0] = NORM ? src[i] * inv * nw[i] : src[i];
+        }
+    };
+    float mx = 0.0f;
+    for (size_t i = (size_t)VE * t; i < k; i += (size_t)VE * NT) {
+        float xn[VE];
+        xnorm(i, xn);
+#pragma unroll
+        for (int e = 0; e < VE; ++e) {
+            const float av = fabsf(xn[e]);
+            if (av > mx) mx = av;
+        }
+    }
+    mx = wave_max<64>(mx);
+    if ((t & 63) == 0) s_max[t >> 6] = mx;
+    __syncthreads();
+    mx = s_max[0];
+#pragma unroll
+    for (int i = 1; i < NT / 64; ++i) mx = fmaxf(mx, s_max[i]);
+    const bool zero = __builtin_isnan(mx) || mx < 1e-12f;
+    const float scale = zero ? 1.0f / 127.0f : mx / 127.0f;
+    for (size_t i = (size_t)VE * t; i < k; i += (size_t)VE * NT) {
+        float xn[VE];
+        int c[VE];
+        xnorm(i, xn);
+#pragma unroll
+        for (int e = 0; e < VE; ++e) c[e] = zero ? 0 : rust_round_clamp_i8(xn[e] / scale, -128.0f, 127.0f);
+        if constexpr (V4)
+            *reinterpret_cast<uint32_t *>(dst + i) = (uint32_t)(c[0] & 255) | ((uint32_t)(c[1] & 255) << 8) |
+                                                     ((uint32_t)(c[2] & 255) << 16) | ((uint32_t)(c[3] & 255) << 24);
+        else dst[i] = (int8_t)c[0];
+    }
+    if (t == 0) *scale_out = scale;
+}
+
+// quantize_absmax_i8 (lib.rs:1072-1098) per row, one workgroup each: a wave for short rows, of which thousands come
+// at once, up to sixteen where a row is long enough to keep them reading. Two passes over the row bound
+// it. (us, 64 / 256 / 1024 threads, launched back to back: 8192 x 256 6.6 / 7.1 / 25, 8192 x 2560 29 / 23 /
+// 38, 1 x 14336 32 / 9.9 / 7.0, 2048 x 14336 59 / 41 / 34)
+template <bool V4, int NT>
+__global__ __launch_bounds__(NT) void absmax_i8_kernel(const float *__restrict__ x, size_t k, int8_t *__restrict__ q,
+                                                       float *__restrict__ scales) {
+    const size_t row = blockIdx.x;
+    absmax_codes<V4, false, NT>(x + row * k, nullptr, 1.0f, k, q + row * k, scales + row);
+}
+
+// subln_quantize_absmax_i8 (lib.rs:1042-1101) per row, one workgroup each.
 //
-// With the norm, the sum of squares is the reference's sequential f32 sum
+// The sum of squares is the reference's sequential f32 sum
 // (dot_product_f32_scalar, lib.rs:770-778): k additions that each wait for the one before, about 9
 // cycles each (26 us for 6912). It is put together in parallel instead, bit for bit: while the
 // running sum stays inside one binade it is an integer A times its ulp u, and adding x >= 0 gives
@@ -385,109 +448,73 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
     return fits ? __uint_as_float(bits) : ordered_sum(acc0, sq, n);
 }
 
-// V4: k % 4 == 0 and 16-byte aligned rows and norm weights (the codes are then stored 4 at a time)
 // PER: squares per thread of a piece (odd, see parallel_ordered_sum); a row longer than PER values per
 // thread is summed in pieces of 14 per thread
 template <bool V4, int PER>
-__global__ __launch_bounds__(kAbsThreads) void absmax_i8_kernel(const float *__restrict__ x,
+__global__ __launch_bounds__(kAbsThreads) void absmax_i8_norm_kernel(const float *__restrict__ x,
                                                                 const float *__restrict__ nw, size_t k, float eps,
                                                                 int8_t *__restrict__ q, float *__restrict__ scales) {
     constexpr int NT = kAbsThreads, VE = V4 ? 4 : 1;
     __shared__ __align__(16) float s_sq[kSqMax];
     __shared__ __align__(16) SumLds s_sum;
     __shared__ float s_inv;
-    __shared__ float s_max[NT / 64];
     const size_t row = blockIdx.x;
     const float *src = x + row * k;
     const int t = threadIdx.x;
-    float inv = 1.0f;
-    if (nw) {
-        float sum_sq = 0.0f;  // (the first wave's)
-        for (size_t c0 = 0; c0 < k; c0 += kSqMax) {
-            const int len = (int)min((size_t)kSqMax, k - c0);
-            if (c0 > 0) {
-                if (t == 0) s_inv = sum_sq;
-                __syncthreads();  // the piece before is summed; its running sum is every thread's
-                sum_sq = s_inv;
-            }
-            for (int i = VE * t; i < len; i += VE * NT) {
-                if constexpr (V4) {
-                    const float4 v = *reinterpret_cast<const float4 *>(src + c0 + i);
-                    *reinterpret_cast<float4 *>(s_sq + i) = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
-                } else {
-                    const float v = src[c0 + i];
-                    s_sq[i] = v * v;
-                }
-            }
-            __syncthreads();
-            if (len <= kSqSerial) sum_sq = t < 64 ? ordered_sum(sum_sq, s_sq, len) : 0.0f;
-            else sum_sq = parallel_ordered_sum<PER>(sum_sq, s_sq, len, s_sum);
+    float sum_sq = 0.0f;  // (the first wave's)
+    for (size_t c0 = 0; c0 < k; c0 += kSqMax) {
+        const int len = (int)min((size_t)kSqMax, k - c0);
+        if (c0 > 0) {
+            if (t == 0) s_inv = sum_sq;
+            __syncthreads();  // the piece before is summed; its running sum is every thread's
+            sum_sq = s_inv;
         }
-        if (t == 0) {
-            const float mean_sq = sum_sq / (float)k;
-            s_inv = 1.0f / sqrtf(mean_sq + eps);
+        for (int i = VE * t; i < len; i += VE * NT) {
+            if constexpr (V4) {
+                const float4 v = *reinterpret_cast<const float4 *>(src + c0 + i);
+                *reinterpret_cast<float4 *>(s_sq + i) = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
+            } else {
+                const float v = src[c0 + i];
+                s_sq[i] = v * v;
+            }
         }
         __syncthreads();
-        inv = s_inv;
+        if (len <= kSqSerial) sum_sq = t < 64 ? ordered_sum(sum_sq, s_sq, len) : 0.0f;
+        else sum_sq = parallel_ordered_sum<PER>(sum_sq, s_sq, len, s_sum);
     }
-    // x_norm of elements i .. i + VE - 1
-    auto xnorm = [&](size_t i, float (&o)[VE]) {
-        if constexpr (V4) {
-            const float4 v = *reinterpret_cast<const float4 *>(src + i);
-            o[0] = v.x, o[1] = v.y, o[2] = v.z, o[3] = v.w;
-            if (nw) {
-                const float4 g = *reinterpret_cast<const float4 *>(nw + i);
-                o[0] = o[0] * inv * g.x, o[1] = o[1] * inv * g.y, o[2] = o[2] * inv * g.z, o[3] = o[3] * inv * g.w;
-            }
-        } else {
-            o[0] = nw ? src[i] * inv * nw[i] : src[i];
-        }
-    };
-    float mx = 0.0f;
-    for (size_t i = (size_t)VE * t; i < k; i += (size_t)VE * NT) {
-        float xn[VE];
-        xnorm(i, xn);
-#pragma unroll
-        for (int e = 0; e < VE; ++e) {
-            const float av = fabsf(xn[e]);
-            if (av > mx) mx = av;
-        }
+    if (t == 0) {
+        const float mean_sq = sum_sq / (float)k;
+        s_inv = 1.0f / sqrtf(mean_sq + eps);
     }
-    mx = wave_max<64>(mx);
-    if ((t & 63) == 0) s_max[t >> 6] = mx;
     __syncthreads();
-    mx = s_max[0];
-#pragma unroll
-    for (int i = 1; i < NT / 64; ++i) mx = fmaxf(mx, s_max[i]);
-    int8_t *dst = q + row * k;
-    const bool zero = __builtin_isnan(mx) || mx < 1e-12f;
-    const float scale = zero ? 1.0f / 127.0f : mx / 127.0f;
-    for (size_t i = (size_t)VE * t; i < k; i += (size_t)VE * NT) {
-        float xn[VE];
-        int c[VE];
-        xnorm(i, xn);
-#pragma unroll
-        for (int e = 0; e < VE; ++e) c[e] = zero ? 0 : rust_round_clamp_i8(xn[e] / scale, -128.0f, 127.0f);
-        if constexpr (V4)
-            *reinterpret_cast<uint32_t *>(dst + i) = (uint32_t)(c[0] & 255) | ((uint32_t)(c[1] & 255) << 8) |
-                                                     ((uint32_t)(c[2] & 255) << 16) | ((uint32_t)(c[3] & 255) << 24);
-        else dst[i] = (int8_t)c[0];
-    }
-    if (t == 0) scales[row] = scale;
+    absmax_codes<V4, true, NT>(src, nw, s_inv, k, q + row * k, scales + row);
+}
+
+template <bool V4>
+static void launch_absmax_plain(hipStream_t s, const float *x, size_t m, size_t k, int8_t *q, float *scales) {
+    const dim3 grid((unsigned)m);
+    if (k <= 1024) hipLaunchKernelGGL((absmax_i8_kernel<V4, 64>), grid, dim3(64), 0, s, x, k, q, scales);
+    else if (k <= 4096) hipLaunchKernelGGL((absmax_i8_kernel<V4, 256>), grid, dim3(256), 0, s, x, k, q, scales);
+    else hipLaunchKernelGGL((absmax_i8_kernel<V4, 1024>), grid, dim3(1024), 0, s, x, k, q, scales);
+}
+
+template <bool V4>
+static void launch_absmax_norm(hipStream_t s, const float *x, const float *nw, size_t m, size_t k, float eps, int8_t *q,
+                               float *scales) {
+    auto launch = [&](auto per) {
+        hipLaunchKernelGGL((absmax_i8_norm_kernel<V4, decltype(per)::value>), dim3((unsigned)m), dim3(kAbsThreads), 0, s, x,
+                           nw, k, eps, q, scales);
+    };
+    if (k <= 3 * kAbsThreads) launch(std::integral_constant<int, 3>());
+    else if (k <= 7 * kAbsThreads) launch(std::integral_constant<int, 7>());
+    else launch(std::integral_constant<int, 15>());
 }
 
 jk_status launch_absmax_i8(hipStream_t s, const float *x, const float *norm_w, size_t m, size_t k, float eps,
                            int8_t *q, float *scales) {
     const bool v4 = k % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)norm_w % 16 == 0 && (uintptr_t)q % 4 == 0;
-    auto launch = [&](auto per) {
-        constexpr int PER = decltype(per)::value;
-        const dim3 grid((unsigned)m), block(kAbsThreads);
-        if (v4) hipLaunchKernelGGL((absmax_i8_kernel<true, PER>), grid, block, 0, s, x, norm_w, k, eps, q, scales);
-        else hipLaunchKernelGGL((absmax_i8_kernel<false, PER>), grid, block, 0, s, x, norm_w, k, eps, q, scales);
-    };
-    if (k <= 3 * kAbsThreads) launch(std::integral_constant<int, 3>());
-    else if (k <= 7 * kAbsThreads) launch(std::integral_constant<int, 7>());
-    else launch(std::integral_constant<int, 15>());
+    if (norm_w) (v4 ? launch_absmax_norm<true> : launch_absmax_norm<false>)(s, x, norm_w, m, k, eps, q, scales);
+    else (v4 ? launch_absmax_plain<true> : launch_absmax_plain<false>)(s, x, m, k, q, scales);
     return check_launch("absmax_i8_kernel");
 }
 

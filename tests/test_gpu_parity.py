@@ -193,6 +193,30 @@ def test_subln_absmax_sizes(gpu, k, offset):
         assert same_bits(host(ds, np.float32, m)[r:r + 1], np.float32([s])), r
 
 
+@pytest.mark.parametrize("m", [3, 300, 1030])
+@pytest.mark.parametrize("k", [5, 64, 256, 257, 1024, 1025, 2051, 3072, 4096, 4100, 7169])
+def test_absmax_rows_and_sizes(gpu, m, k):
+    """Both absmax quantizers at few rows, more rows than CUs and more than four times as many, on both sides of
+    the row lengths where the launch changes, aligned and not, in one piece and several: normal rows, rows of bf16 values (whose squares lie between two
+    ulps of the running sum again and again) and mostly-zero rows, equal to the oracle."""
+    torch = gpu
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[1::3] = torch.from_numpy(x[1::3]).bfloat16().float().numpy()
+    x[2::3][rng.random(x[2::3].shape) < 0.9] = 0
+    w = rng.uniform(0.5, 1.5, k).astype(np.float32)
+    dx, dw = dev(torch, x), dev(torch, w)
+    dq, ds, dq2, ds2 = empty(torch, m * k), empty(torch, 4 * m), empty(torch, m * k), empty(torch, 4 * m)
+    jk.dev_subln_quantize_absmax_i8(dx, dw, m, k, 1e-5, dq, ds)
+    jk.dev_quantize_absmax_i8(dx, m, k, dq2, ds2)
+    torch.cuda.synchronize()
+    for codes, scales, ref in ((dq, ds, [O.subln_quantize_absmax_i8(r, w, 1e-5) for r in x]),
+                               (dq2, ds2, [O.quantize_absmax_i8(r) for r in x])):
+        want = np.float32([s for _, s in ref])
+        assert same_bits(host(scales, np.float32, m), want), mismatch(host(scales, np.float32, m), want)
+        assert np.array_equal(host(codes, np.int8, m * k).reshape(m, k), np.stack([q for q, _ in ref]))
+
+
 @pytest.mark.parametrize("k,per", [(2800, 3), (4859, 7), (7381, 15)])
 def test_subln_absmax_lagging_sum(gpu, k, per):
     """Rows whose ordered sum lags the plain prefix sums from which the parallel form takes each element's
