@@ -1100,7 +1100,7 @@ gemm_q8_0_exact_dma_128(WeightDev w, jk_act_q8 a, float *__restrict__ y, int r0,
     gemm_q8_0_tol_dma<128, true>(w, a, y, r0, r1);
 }
 
-static long cu_count() {
+long cu_count() {
     static long n = 0;
     if (n == 0) {
         int dev = 0, v = 0;

@@ -1101,18 +1101,6 @@ static int resident_per_cu(K kernel, size_t lds, int threads) {
     return n;
 }
 
-static int cu_count() {
-    static int n = 0;
-    if (n == 0) {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-            n = v;
-        else
-            n = 256;
-    }
-    return n;
-}
-
 // The argmax of each argmax job of a launched group: reduce its workgroups' keys.
 static jk_status launch_group_argmax(hipStream_t s, const GemvGroup &g) {
     for (int i = 0; i < g.njobs; ++i)
@@ -1126,7 +1114,7 @@ static jk_status launch_group_run(hipStream_t s, GemvGroup &g, size_t lds) {
     constexpr int RPU = 64 / LPR;
     auto kern = gemv_q8_group_kernel<Q, LPR, F32, NW>;
     // Size the grid to one resident round: each wave then walks ceil(units / waves) units.
-    const int cap_waves = resident_per_cu(kern, lds, 64 * NW) * cu_count() * NW;
+    const int cap_waves = resident_per_cu(kern, lds, 64 * NW) * (int)cu_count() * NW;
     long total = 0;
     for (int i = 0; i < g.njobs; ++i) total += (g.job[i].r1 - g.job[i].r0 + RPU - 1) / RPU;
     // (at most 16 units per wave: bigger jobs get more than one round of workgroups)

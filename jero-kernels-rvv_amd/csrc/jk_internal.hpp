@@ -188,6 +188,7 @@ jk_status dot_i8_check(const int8_t *a, size_t a_len, const int8_t *b, size_t b_
 
 // Checks the last kernel launch on the current thread.
 jk_status check_launch(const char *what);
+long cu_count();  // compute units of the device
 
 // Launch plans: with t_plan.dry set, the GEMM / BitLinear launchers record the kernel they
 // would launch (its name) instead of launching it. jk_gemm_plan / jk_bitlinear_plan use this

@@ -294,7 +294,6 @@ __global__ __launch_bounds__(NT) void absmax_i8_kernel(const float *__restrict__
 // by one thread from global memory). What bounds it now: the three scans' cross-lane steps, the
 // elements added one by one (a scalar round trip each) and three passes over the row.
 constexpr int kAbsThreads = 1024;
-constexpr int kSqMax = 14336;     // squares held in LDS at once (14 per thread); longer rows go in such pieces
 constexpr int kSqSerial = 256;    // pieces up to this length are added one by one
 constexpr int kSqEvents = 256;    // elements added one by one otherwise, at most
 
@@ -307,23 +306,23 @@ struct SumLds {
     int tail_eb;                                     // binade after the last element
 };
 
-// acc + s[0] + s[1] + ... + s[n - 1], in order (s: LDS, the same for every lane; n >= 1). Reads are
-// requested sixteen ahead and unconditional (past the end the last value, replaced by -0.0, the
-// identity of f32 addition): a read behind a test waits for itself.
+// acc + s[0] + s[1] + ... + s[n - 1], in order (s: 16-byte aligned LDS, the same for every lane; up to
+// the next multiple of 32 it holds -0.0, the identity of f32 addition), from 16-byte broadcast reads
+// requested 32 values ahead, so that an addition waits only for the one before it.
 __device__ __forceinline__ float ordered_sum(float acc, const float *s, int n) {
-    constexpr int N = 16;
-    float cur[N], nxt[N];
+    const float4 *s4 = reinterpret_cast<const float4 *>(s);
+    const int n32 = (n + 31) / 32;
+    float4 cur[8], nxt[8];
 #pragma unroll
-    for (int i = 0; i < N; ++i) cur[i] = s[min(i, n - 1)];
-    for (int c = 0; c < n; c += N) {
+    for (int i = 0; i < 8; ++i) cur[i] = s4[i];
+    for (int c = 0; c < n32; ++c) {
+        const int cn = min(c + 1, n32 - 1);
 #pragma unroll
-        for (int i = 0; i < N; ++i) nxt[i] = s[min(c + N + i, n - 1)];
+        for (int i = 0; i < 8; ++i) nxt[i] = s4[8 * cn + i];
 #pragma unroll
-        for (int i = 0; i < N; ++i) cur[i] = c + i < n ? cur[i] : -0.0f;
+        for (int i = 0; i < 8; ++i) acc = (((acc + cur[i].x) + cur[i].y) + cur[i].z) + cur[i].w;
 #pragma unroll
-        for (int i = 0; i < N; ++i) acc += cur[i];
-#pragma unroll
-        for (int i = 0; i < N; ++i) cur[i] = nxt[i];
+        for (int i = 0; i < 8; ++i) cur[i] = nxt[i];
     }
     return acc;
 }
@@ -448,22 +447,23 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
     return fits ? __uint_as_float(bits) : ordered_sum(acc0, sq, n);
 }
 
-// PER: squares per thread of a piece (odd, see parallel_ordered_sum); a row longer than PER values per
-// thread is summed in pieces of 14 per thread
-template <bool V4, int PER>
-__global__ __launch_bounds__(kAbsThreads) void absmax_i8_norm_kernel(const float *__restrict__ x,
-                                                                const float *__restrict__ nw, size_t k, float eps,
-                                                                int8_t *__restrict__ q, float *__restrict__ scales) {
-    constexpr int NT = kAbsThreads, VE = V4 ? 4 : 1;
-    __shared__ __align__(16) float s_sq[kSqMax];
-    __shared__ __align__(16) SumLds s_sum;
+// SQ: values of a row summed at once, in LDS (a multiple of 32; a longer row in such pieces). PER: values per thread
+// of the parallel sum (odd, see above; of 15, 14 are used: a workgroup's squares stay below 64 KB), or 0
+// for the sum in order by the first wave.
+template <bool V4, int NT, int PER, int SQ>
+__global__ __launch_bounds__(NT) void absmax_i8_norm_kernel(const float *__restrict__ x, const float *__restrict__ nw,
+                                                            size_t k, float eps, int8_t *__restrict__ q,
+                                                            float *__restrict__ scales) {
+    static_assert(PER == 0 || (NT == kAbsThreads && SQ <= PER * NT), "the parallel sum's threads");
+    constexpr int VE = V4 ? 4 : 1;
+    __shared__ __align__(16) float s_sq[SQ];
     __shared__ float s_inv;
     const size_t row = blockIdx.x;
     const float *src = x + row * k;
     const int t = threadIdx.x;
     float sum_sq = 0.0f;  // (the first wave's)
-    for (size_t c0 = 0; c0 < k; c0 += kSqMax) {
-        const int len = (int)min((size_t)kSqMax, k - c0);
+    for (size_t c0 = 0; c0 < k; c0 += SQ) {
+        const int len = (int)min((size_t)SQ, k - c0);
         if (c0 > 0) {
             if (t == 0) s_inv = sum_sq;
             __syncthreads();  // the piece before is summed; its running sum is every thread's
@@ -478,9 +478,14 @@ __global__ __launch_bounds__(kAbsThreads) void absmax_i8_norm_kernel(const float
                 s_sq[i] = v * v;
             }
         }
+        if (t < (-len & 31)) s_sq[len + t] = -0.0f;
         __syncthreads();
-        if (len <= kSqSerial) sum_sq = t < 64 ? ordered_sum(sum_sq, s_sq, len) : 0.0f;
-        else sum_sq = parallel_ordered_sum<PER>(sum_sq, s_sq, len, s_sum);
+        if (PER == 0 || len <= kSqSerial) {
+            sum_sq = t < 64 ? ordered_sum(sum_sq, s_sq, len) : 0.0f;
+        } else if constexpr (PER > 0) {
+            __shared__ __align__(16) SumLds s_sum;
+            sum_sq = parallel_ordered_sum<PER>(sum_sq, s_sq, len, s_sum);
+        }
     }
     if (t == 0) {
         const float mean_sq = sum_sq / (float)k;
@@ -498,16 +503,26 @@ static void launch_absmax_plain(hipStream_t s, const float *x, size_t m, size_t 
     else hipLaunchKernelGGL((absmax_i8_kernel<V4, 1024>), grid, dim3(1024), 0, s, x, k, q, scales);
 }
 
+// The parallel sum takes a workgroup per CU and its time is its latency, so it is for as many rows as there are
+// CUs, or few rounds of long ones; more rows go in order, in small workgroups of which a CU holds many
+// (us, launched back to back: 64 threads 8192 x 256 8.8, 8192 x 1000 26, 600 x 1000 9.1; 256 threads 600 x 2560
+// 14.8, 2048 x 2560 18, 2048 x 6912 49; the parallel sum 8192 x 256 219, 8192 x 1000 114, 600 x 1000 13.9, 600 x 2560
+// 15.9, 2048 x 2560 35, 2048 x 6912 82; and 600 x 6912 31 against 34 in order). Rows of up to 256 values
+// are as soon added by one wave as shared out.
 template <bool V4>
 static void launch_absmax_norm(hipStream_t s, const float *x, const float *nw, size_t m, size_t k, float eps, int8_t *q,
                                float *scales) {
-    auto launch = [&](auto per) {
-        hipLaunchKernelGGL((absmax_i8_norm_kernel<V4, decltype(per)::value>), dim3((unsigned)m), dim3(kAbsThreads), 0, s, x,
-                           nw, k, eps, q, scales);
+    const dim3 grid((unsigned)m);
+    const size_t ncu = (size_t)cu_count();
+    auto launch = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, grid, dim3((unsigned)threads), 0, s, x, nw, k, eps, q, scales);
     };
-    if (k <= 3 * kAbsThreads) launch(std::integral_constant<int, 3>());
-    else if (k <= 7 * kAbsThreads) launch(std::integral_constant<int, 7>());
-    else launch(std::integral_constant<int, 15>());
+    constexpr int T = kAbsThreads;
+    if (k <= kSqSerial || (m > ncu && k <= 1024)) launch(absmax_i8_norm_kernel<V4, 64, 0, 1024>, 64);
+    else if (m > ncu && (k <= 4096 || m > 4 * ncu)) launch(absmax_i8_norm_kernel<V4, 256, 0, 2048>, 256);
+    else if (k <= 3 * T) launch(absmax_i8_norm_kernel<V4, T, 3, 3 * T>, T);
+    else if (k <= 7 * T) launch(absmax_i8_norm_kernel<V4, T, 7, 7 * T>, T);
+    else launch(absmax_i8_norm_kernel<V4, T, 15, 14 * T>, T);
 }
 
 jk_status launch_absmax_i8(hipStream_t s, const float *x, const float *norm_w, size_t m, size_t k, float eps,
