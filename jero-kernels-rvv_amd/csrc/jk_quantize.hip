@@ -275,35 +275,80 @@ __global__ __launch_bounds__(NT) void absmax_i8_kernel(const float *__restrict__
 
 // subln_quantize_absmax_i8 (lib.rs:1042-1101) per row, one workgroup each.
 //
-// The sum of squares is the reference's sequential f32 sum
-// (dot_product_f32_scalar, lib.rs:770-778): k additions that each wait for the one before, about 9
-// cycles each (26 us for 6912). It is put together in parallel instead, bit for bit: while the
-// running sum stays inside one binade it is an integer A times its ulp u, and adding x >= 0 gives
-// RNE(A + x / u) u, so A grows by round(x / u) whatever A is -- except where x / u lies exactly
-// between two integers (a tie goes to the even neighbour, which depends on A) or the sum leaves the
-// binade. An approximate prefix sum tells each element's binade; the increments are added by an
-// integer scan; and the elements where the rule does not hold (within 2e-5 of a power of two, about
-// one per doubling of the sum; ties; the first element; NaN and Inf; sums near the ends of the
-// exponent range) are added one by one by the first wave, between them the scan's increments as one
-// integer addition to the float's bits. That addition is checked to start and to end in the
-// expected binade, and all its elements to have been given that binade (a thread's approximate prefix
-// can lie a few ulps below the end of the thread before it, put together in another order, and fall
-// back into the binade below); where a check fails, or with too many such elements, the first wave adds
-// the whole row one by one. Normal rows of 2560 and 6912 have 21 and 23 such elements: 7.8 and 10.5 us a
-// launch, against 12.7 and 29.3 us with every element added from LDS by the first wave (about 190 us
-// by one thread from global memory). What bounds it now: the three scans' cross-lane steps, the
-// elements added one by one (a scalar round trip each) and three passes over the row.
+// The sum of squares is the reference's sequential f32 sum (dot_product_f32_scalar, lib.rs:770-778):
+// k additions that each wait for the one before, about 7 cycles each from LDS (20 us for 6912; 190 us by
+// one thread from global memory). For few rows it is put together in parallel instead, bit for bit: while
+// the running sum stays inside one binade it is an integer A times its ulp u, and adding x >= 0 gives
+// RNE(A + x / u) u: A grows by round(x / u), where a tie goes to the even neighbour and so depends on
+// whether A is even. What a run of elements adds is therefore a pair of integers, for A even and for A
+// odd, and pairs are put together by a scan. (Ties are common: squares of bf16 values have few low
+// bits.) An approximate prefix sum tells each element's binade. The elements where the rule does not
+// hold (within 2e-5 of a power of two, about one per doubling of the sum; the first element; NaN and
+// Inf; sums near the ends of the exponent range) are added one by one by the first wave, between them
+// the runs, each as one integer addition to the float's bits. That addition is checked to start and to
+// end in the expected binade, and all its elements to have been given that binade (a thread's
+// approximate prefix can lie a few ulps below the end of the thread before it, put together in another
+// order, and fall back into the binade below); where a check fails, or with too many elements outside
+// the rule, the first wave adds the whole row in order. Normal rows of 2560 and 6912 have 12 and 14 such
+// elements, of f32 and of bf16 values alike: 7.6 and 10.8 us a launch (with every tie added one by one
+// 8.2 and 11 us, and for bf16 values, 325 and 726 ties, 60 and 152 us). What bounds it now: the scans'
+// cross-lane steps, the elements added one by one (a scalar round trip each) and three passes over the row.
 constexpr int kAbsThreads = 1024;
 constexpr int kSqSerial = 256;    // pieces up to this length are added one by one
-constexpr int kSqEvents = 256;    // elements added one by one otherwise, at most
+constexpr int kSqEvents = 256;    // elements outside the rule, at most
+
+// What adding a run of elements adds to the running sum's integer A, for A even and for A odd.
+struct SumRun {
+    int even, odd;
+};
+__device__ __forceinline__ SumRun run_then(SumRun f, SumRun g) {
+    return {f.even + ((f.even & 1) ? g.odd : g.even), f.odd + ((f.odd & 1) ? g.even : g.odd)};
+}
+
+// Inclusive scans over the lanes of a 16-lane row (WAVE: of the wave) by DPP moves, whose lanes without a
+// source get zeros, the identity of all three.
+template <int CTRL, int ROWS = 0xF> __device__ __forceinline__ int dpp_or0(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+template <bool WAVE> __device__ __forceinline__ float scan_add(float v) {
+    auto f = [](int x) { return __int_as_float(x); };
+    v += f(dpp_or0<0x111>(__float_as_int(v)));  // row_shr:1, 2, 4, 8
+    v += f(dpp_or0<0x112>(__float_as_int(v)));
+    v += f(dpp_or0<0x114>(__float_as_int(v)));
+    v += f(dpp_or0<0x118>(__float_as_int(v)));
+    if constexpr (WAVE) {
+        v += f(dpp_or0<0x142, 0xA>(__float_as_int(v)));  // row_bcast:15 into rows 1 and 3
+        v += f(dpp_or0<0x143, 0xC>(__float_as_int(v)));  // row_bcast:31 into rows 2 and 3
+    }
+    return v;
+}
+// run: since the last of cnt events
+template <int CTRL, int ROWS = 0xF> __device__ __forceinline__ void scan_run_step(SumRun &run, int &cnt) {
+    const SumRun r = run_then({dpp_or0<CTRL, ROWS>(run.even), dpp_or0<CTRL, ROWS>(run.odd)}, run);
+    const int c = dpp_or0<CTRL, ROWS>(cnt);
+    run = cnt ? run : r;
+    cnt += c;
+}
+template <bool WAVE> __device__ __forceinline__ void scan_runs(SumRun &run, int &cnt) {
+    scan_run_step<0x111>(run, cnt);
+    scan_run_step<0x112>(run, cnt);
+    scan_run_step<0x114>(run, cnt);
+    scan_run_step<0x118>(run, cnt);
+    if constexpr (WAVE) {
+        scan_run_step<0x142, 0xA>(run, cnt);
+        scan_run_step<0x143, 0xC>(run, cnt);
+    }
+}
 
 struct SumLds {
-    float part[kAbsThreads / 64];                    // per wave: sum of its squares
-    int inc[kAbsThreads / 64], cnt[kAbsThreads / 64];  // increments and events
-    int4 ev[kSqEvents];                              // position, increments before it, binade, the square's bits
-    uint32_t first[kAbsThreads / 64], last[kAbsThreads / 64];  // binades of the wave's first and last elements
-    int split[kAbsThreads / 64];                     // whether a run changes its binade between two threads of the wave
-    int tail_eb;                                     // binade after the last element
+    static constexpr int NW = kAbsThreads / 64;
+    float part[NW];                  // per wave: sum of its squares
+    SumRun run[NW];                  // and its run after its last event, and its events
+    int cnt[NW];
+    uint32_t first[NW], last[NW];    // binades of the wave's first and last elements
+    int split[NW];                   // whether a run changes its binade between two threads of the wave
+    int4 ev[kSqEvents];              // position and binade, the run before it, the square's bits
+    int tail_eb;                     // binade after the last element
 };
 
 // acc + s[0] + s[1] + ... + s[n - 1], in order (s: 16-byte aligned LDS, the same for every lane; up to
@@ -332,7 +377,8 @@ __device__ __forceinline__ float ordered_sum(float acc, const float *s, int n) {
 template <int PER>
 __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *sq, int n, SumLds &L) {
     constexpr int NW = kAbsThreads / 64;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    static_assert(NW <= 16, "the waves' values in one row");
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int lo = t * PER;
     float v[PER];
 #pragma unroll
@@ -343,28 +389,24 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
         v[i] = lo + i < n ? v[i] : 0.0f;
         part += v[i];
     }
-    float incl = part;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const float u = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += u;
-    }
+    const float incl = scan_add<true>(part);
     if (lane == 63) L.part[wave] = incl;
     __syncthreads();
-    float pre = acc0 + (incl - part);  // approximate sum before the thread's first element
-#pragma unroll
-    for (int i = 0; i < NW; ++i) pre += i < wave ? L.part[i] : 0.0f;
-    // element i after an approximate sum p: its binade, whether it goes by the rule, and its increment
+    const float waves = scan_add<false>(lane < NW ? L.part[lane] : 0.0f);
+    const float before_wave = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(waves), max(wave - 1, 0)));
+    const float pre = acc0 + (wave > 0 ? before_wave : 0.0f) + (incl - part);  // approximate sum before the thread
+    // element i after an approximate sum p: its binade, whether it goes by the rule, and its increments
     auto element = [&](int i, float p, uint32_t &eb, bool &ok) {
         eb = __float_as_uint(p * 0.99998f) >> 23;
         const uint32_t ee = __float_as_uint((p + v[i]) * 1.00002f) >> 23;
         const float to_ulp = __uint_as_float((277u - min(max(eb, 30u), 220u)) << 23);  // 1 / u, a power of two
         const float w = v[i] * to_ulp, fl = floorf(w), fr = w - fl;
-        ok = eb == ee && eb >= 30 && eb <= 220 && w < 16777216.0f && fr != 0.5f;
-        return ok ? (int)fl + (fr > 0.5f ? 1 : 0) : 0;
+        ok = eb == ee && eb >= 30 && eb <= 220 && w < 16777216.0f;
+        const int b = (int)fl, up = fr > 0.5f, tie = fr == 0.5f;
+        return ok ? SumRun{b + (up | (tie & b)), b + (up | (tie & ~b))} : SumRun{0, 0};
     };
     uint32_t events = 0;
-    int inc = 0;
+    SumRun run = {0, 0};  // since the last event
     float p = pre;
     uint32_t first = 0, last = 0;  // binades of the first and the last element (kNoRun: no run goes on past it)
     constexpr uint32_t kNoRun = 1u << 16;
@@ -372,10 +414,11 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
     for (int i = 0; i < PER; ++i) {
         uint32_t eb;
         bool ok;
-        const int r = element(i, p, eb, ok);
+        const SumRun r = element(i, p, eb, ok);
         p += v[i];
         const bool live = lo + i < n;
-        inc += live ? r : 0;
+        const SumRun next = run_then(run, r);
+        run = live ? (ok ? next : SumRun{0, 0}) : run;
         events |= (uint32_t)(live && !ok) << i;
         if (lo + i == n - 1) L.tail_eb = (int)eb;
         if (i == 0) first = live ? eb : kNoRun;
@@ -383,67 +426,68 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
     }
     // the elements of a run share a binade: within a thread by construction (an element by the rule ends in
     // the binade that the next one starts from), from one thread to the next by this test
-    const uint32_t before = __shfl_up(last, 1, 64);
+    const uint32_t before = (uint32_t)dpp_or0<0x138>((int)last);  // wave_shr:1
     const bool split = lane > 0 && ((before | first) & kNoRun) == 0 && before != first;
     const uint64_t any_split = __ballot(split);
     if (lane == 0) L.first[wave] = first, L.split[wave] = any_split != 0;
     if (lane == 63) L.last[wave] = last;
-    int pi = inc, pc = __popc(events);
-    const int cnt = pc;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int ui = __shfl_up(pi, o, 64), uc = __shfl_up(pc, o, 64);
-        if (lane >= o) pi += ui, pc += uc;
-    }
-    if (lane == 63) L.inc[wave] = pi, L.cnt[wave] = pc;
+    const int cnt = __popc(events);
+    int pc = cnt;
+    scan_runs<true>(run, pc);
+    if (lane == 63) L.run[wave] = run, L.cnt[wave] = pc;
+    const SumRun ex = {dpp_or0<0x138>(run.even), dpp_or0<0x138>(run.odd)};  // before the thread, in its wave
     __syncthreads();
-    int ri = pi - inc, ci = pc - cnt, total_i = 0, total_c = 0;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-        ri += i < wave ? L.inc[i] : 0, ci += i < wave ? L.cnt[i] : 0;
-        total_i += L.inc[i], total_c += L.cnt[i];
-    }
+    SumRun wr = lane < NW ? L.run[lane] : SumRun{0, 0};
+    int wc = lane < NW ? L.cnt[lane] : 0;
+    scan_runs<false>(wr, wc);
+    const int prev = max(wave - 1, 0);
+    const SumRun wp = {__builtin_amdgcn_readlane(wr.even, prev), __builtin_amdgcn_readlane(wr.odd, prev)};
+    const int before_c = __builtin_amdgcn_readlane(wc, prev), total_c = __builtin_amdgcn_readlane(wc, NW - 1);
     if (events) {
+        int ci = (wave > 0 ? before_c : 0) + pc - cnt;
+        run = pc > cnt || wave == 0 ? ex : run_then(wp, ex);
         p = pre;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             uint32_t eb;
             bool ok;
-            const int r = element(i, p, eb, ok);
+            const SumRun r = element(i, p, eb, ok);
             p += v[i];
-            if ((events >> i) & 1u) {
-                if (ci < kSqEvents) L.ev[ci] = make_int4(lo + i, ri, (int)eb, __float_as_int(v[i]));
-                ++ci;
-            }
-            ri += r;
+            const bool event = (events >> i) & 1u;
+            if (event && ci < kSqEvents)
+                L.ev[ci] = make_int4((lo + i) << 9 | (int)eb, run.even, run.odd, __float_as_int(v[i]));
+            ci += event;
+            const SumRun next = run_then(run, r);
+            run = event ? SumRun{0, 0} : next;
         }
     }
     __syncthreads();
     if (t >= 64) return 0.0f;
     uint32_t bits = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(acc0));
-    bool fits = total_c <= kSqEvents;
-    for (int i = 0; i < NW; ++i) {
-        fits = fits && !L.split[i];
-        if (i > 0) fits = fits && (((L.last[i - 1] | L.first[i]) & kNoRun) != 0 || L.last[i - 1] == L.first[i]);
-    }
-    int pos = -1, done = 0;  // the last element added, and the increments added (scalars)
-    // the increments up to (not including) element p, all in binade e
-    auto advance = [&](int p, int upto, uint32_t e) {
-        const uint32_t to = bits + (uint32_t)(upto - done);
+    const int w1 = min(lane, NW - 1), w0 = max(w1 - 1, 0);
+    const uint32_t l0 = L.last[w0], f1 = L.first[w1];
+    const bool gap = L.split[w1] || (w1 > 0 && ((l0 | f1) & kNoRun) == 0 && l0 != f1);
+    bool fits = total_c <= kSqEvents && __ballot(gap) == 0;
+    const SumRun tail = {__builtin_amdgcn_readlane(wr.even, NW - 1), __builtin_amdgcn_readlane(wr.odd, NW - 1)};
+    int pos = -1;  // the last element added (scalars)
+    // the run up to (not including) element p, all in binade e
+    auto advance = [&](int p, int even, int odd, uint32_t e) {
+        const uint32_t to = bits + (uint32_t)((bits & 1u) ? odd : even);
         if (p > pos + 1 && ((bits >> 23) != e || (to >> 23) != e)) fits = false;
-        bits = to, done = upto;
+        bits = to;
     };
     for (int g = 0; fits && g < total_c; g += 64) {
         const int4 ev = L.ev[min(g + lane, total_c - 1)];  // lane l: event g + l
         for (int j = 0; j < min(64, total_c - g); ++j) {
-            const int p = __builtin_amdgcn_readlane(ev.x, j);
-            advance(p, __builtin_amdgcn_readlane(ev.y, j), (uint32_t)__builtin_amdgcn_readlane(ev.z, j));
+            const uint32_t at = (uint32_t)__builtin_amdgcn_readlane(ev.x, j);
+            const int p = (int)(at >> 9);
+            advance(p, __builtin_amdgcn_readlane(ev.y, j), __builtin_amdgcn_readlane(ev.z, j), at & 511u);
             const float acc = __uint_as_float(bits) + __int_as_float(__builtin_amdgcn_readlane(ev.w, j));
             bits = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(acc));
             pos = p;
         }
     }
-    advance(n, total_i, (uint32_t)__builtin_amdgcn_readfirstlane(L.tail_eb));
+    advance(n, tail.even, tail.odd, (uint32_t)__builtin_amdgcn_readfirstlane(L.tail_eb));
     return fits ? __uint_as_float(bits) : ordered_sum(acc0, sq, n);
 }
 
