@@ -2096,48 +2096,89 @@ static jk_status launch_gemm_tol(hipStream_t s, const WeightDev &w, const jk_act
     }
 }
 
-// Whether a launch of 3 or more tokens takes jk_gemm_few.hip's kernel (the formats and layouts it has).
-// Bit-exact: wherever the tiled launch would leave the 128 x 64 tiles, down to where those smaller tiles
-// have waves enough -- 64 x 64 tiles at more than 2.75 per CU (Q8_0: 2.25), 32 x 32 ones at more than
-// 6 per CU for Q5_K and Q6_K, whose unpacking the small tiles repeat more often. Measured (us, 4096
-// columns, new against tiled): Q4_K 14336 rows 8 / 100 / 192 / 256 tokens 16 / 65 / 93 / 110 against
-// 39 / 73 / 99 / 109, 4096 rows 4 / 50 / 512 / 900 tokens 8 / 13 / 64 / 121 against 34 / 38 / 94 /
-// 108; Q8_0 14336 rows 4 / 100 / 160 tokens 16 / 53 / 78 against 31 / 57 / 72; Q5_K 14336 rows 40 /
-// 128 tokens 33 / 90 against 59 / 86; Q6_K 14336 rows 40 / 100 tokens 56 / 92 against 66 / 89,
-// 4096 x 14336 at 4 / 512 / 768 tokens 26 / 334 / 496 against 201 / 437 / 445.
-// Tolerance mode: up to four 16 x 16 tiles per CU, where splitting K over four waves of a workgroup
-// repeats its loads and unpacking for tokens that are not there (Q4_K 14336 rows 8 tokens 14 against
-// 22, 4096 rows 50 tokens 11 against 19; Q6_K 4096 x 14336 64 tokens 46 against 78); 33 to 48 tokens
-// of the 32-element-group formats, which that kernel pads to 64 (14336 rows 27 against 30); and
-// where the tolerance launch would run the bit-exact tiles (4096 rows 600 tokens 71 against 96).
+// Whether a launch of 3 or more tokens takes jk_gemm_few.hip's kernel (the formats and layouts it has),
+// from some 15,000 shapes of 64 to 128256 rows, 512 to 14336 columns and 3 to 2048 tokens timed on both
+// sides. Its time grows by whole rounds of one workgroup per CU, so the limits are in workgroups W, as
+// it would launch them, per CU. Bit-exact:
+// * up to ten 16 x 16 tiles per CU, where it splits K: 0.11 to 1.0 of the tiled launch (us, 4096
+//   columns, new against tiled: Q4_K 4096 rows 4 / 50 tokens 8 / 13 against 34 / 38);
+// * beyond, against 32 x 32 tiles and up to 2.75 64 x 64 tiles per CU (Q8_0 2.25; not swept further but
+//   for a vocabulary's rows at up to 32 tokens, where Q5_K and Q6_K, left there, took 0.4 of the tiled
+//   time). Q8_0: one round (14336 rows 41 tokens 23 against 39), or two that are two thirds full (4050
+//   x 14336, 485 tokens 164 against 217; 5875 x 8192, 160 tokens (0.45) 93 against 76), with 33 to 48
+//   tokens any two (25011 x 1024 14 against 17). Q4_0: three rounds (8192 x 8192, 183 tokens 81 against
+//   98), not part of a fourth against 32 x 32 tiles (14336 rows 102 tokens 55 against 53; below 2048
+//   columns yes: 4553 x 1024, 415 tokens 17.7 against 19.5), up to five (11008 rows 150 tokens 54
+//   against 71, 14336 rows 131 tokens 69 against 73), not more (171 tokens 81 against 71); of 33 to 48
+//   tokens two (24093 x 1024 15 against 17; 63141 rows, four, 93 against 78), of 49 to 64 one (24370
+//   rows, two, 57 against 51). Q5_K: below 2048 columns three rounds against 32 x 32 tiles (4178 x 768,
+//   378 tokens, in four, 22 against 20), four (1169 x 14336, 1312 tokens 276 against 295; 8192 x 8192,
+//   208 tokens 160 against 188), in tolerance mode five (14336 rows 159 tokens 94 against 104), not six
+//   (162 tokens 123 against 103; tolerance 112 against 104). Q6_K: six, against 64 x 64 tiles ten
+//   (14336 rows 132 tokens 114 against 132), not eleven (169 tokens 135 against 129) but of up to 64
+//   tokens (43583 x 2048, 40 tokens 77 against 98). Q4_K: any (14336 rows 164 tokens 91 against 96).
+// Tolerance mode, whose sums need no order, so that the launch below splits K too:
+// * up to four 16 x 16 tiles per CU, as that launch repeats its loads and unpacking for tokens that are
+//   not there (Q4_K 4096 rows 50 tokens 11 against 19, Q6_K 4096 x 14336 64 tokens 46 against 78), not
+//   in a second round of the four-tile workgroups (Q8_0 4197 rows 44 tokens 17 against 14);
+// * 33 to 48 tokens of the 32-element-group formats, which that kernel pads to 64 (Q8_0 14336 x 2048,
+//   47 tokens 12.0 against 13.6), in one round, or in more than one and a half (Q8_0 29444 x 1024, 36
+//   tokens 13 against 16, Q4_K 45411 x 2048, 41 tokens 41 against 63; one and a quarter 1.16 of its
+//   time), below eleven 16 x 16 tiles in three rounds of Q4_K and Q5_K (8633 x 1536, 44 tokens 13
+//   against 14); Q4_0 in one round only below 2048 columns (14336 x 1024 8.0 against 8.8, x 4096 23.8
+//   against 21.2); or where 128 x 128 tiles would pad them to 128 (Q4_K 54220 x 2048, 48 tokens 53
+//   against 85);
+// * where the tolerance launch would run the bit-exact tiles, by the limits above.
 static bool few_better(const WeightDev &w, const jk_act_q8 &a, long rows, bool tol) {
     if (!gemm_few_ok(w, a)) return false;
     const long ncu = cu_count(), m = (long)a.m;
-    auto tiles = [&](long t) { return (rows + t - 1) / t * ((m + t - 1) / t); };
-    const int tile = gemm_tile(w.quant, rows, m);
+    auto tiles = [&](long tn, long tm) { return (rows + tn - 1) / tn * ((m + tm - 1) / tm); };
+    const long t16 = tiles(16, 16), W = gemm_few_workgroups(w.quant, rows, m, ncu);
+    const int q = w.quant, tile = gemm_tile(q, rows, m);
+    const bool three = m > 32 && m <= 48;  // token tiles of 16: unsplit, one workgroup's
     if (tol && w.cols % 128 == 0) {
-        if (tiles(16) <= 4 * ncu || (m > 32 && m <= 48 && w.quant != JK_Q6_K)) return true;
-        if (tile != 1 || w.quant == JK_Q6_K || 2 * tiles(128) >= 3 * ncu) return false;
+        if (t16 <= 4 * ncu) return m <= 32 || t16 <= 2 * ncu || W <= ncu;
+        const bool wide = 2 * tiles(128, 128) >= 3 * ncu;  // the launch below runs 128 x 128 tiles
+        if (three && t16 > 10 * ncu && q != JK_Q6_K)
+            return wide || (q == JK_Q4_0 ? W > 2 * ncu || (W <= ncu && w.cols < 2048) : W <= ncu || 2 * W > 3 * ncu);
+        if (three && t16 <= 10 * ncu && (q == JK_Q4_K || q == JK_Q5_K)) return W <= 3 * ncu;
+        if (tile != 1 || q == JK_Q6_K || wide) return false;
     }
-    switch (tile) {
-    case 0: return false;
-    case 1: return 4 * tiles(64) <= (w.quant == JK_Q8_0 ? 9 : 11) * ncu;
-    default: return w.quant == JK_Q4_K || w.quant == JK_Q4_0 || w.quant == JK_Q8_0 || tiles(32) <= 6 * ncu;
+    if (tile == 0) return false;
+    if (t16 <= 10 * ncu) return true;
+    if (tile == 1 && 4 * tiles(64, 64) > (q == JK_Q8_0 ? 9 : 11) * ncu) return false;
+    switch (q) {
+    case JK_Q8_0: return W <= ncu || (W <= 2 * ncu && (three || 3 * rows * m >= 4 * 64 * 64 * ncu));
+    case JK_Q4_0:
+        if (m > 32 && m <= 64) return W <= (three ? 2 : 1) * ncu;
+        return W <= (w.cols < 2048 ? 4 : 3) * ncu || ((tile == 1 || 4 * W > 15 * ncu) && W <= 5 * ncu);
+    case JK_Q5_K: return W <= (tile == 2 && w.cols < 2048 ? 3 : tol ? 5 : 4) * ncu;
+    case JK_Q6_K: return W <= (tile == 2 ? 6 : m <= 64 ? 11 : 10) * ncu;
+    default: return true;  // Q4_K
     }
 }
 
 // Whether a tolerance-mode launch takes jk_gemm_split.hip's kernel: its tiles of 256 rows x 128 tokens
 // cost the same whether full or not and run one to a CU, so the outputs have to fill half of the rounds
 // that the tiles need. Measured (us, new against the launches below): Q4_K x 4096 columns, 11008 rows
-// 384 tokens (0.5 of one round) 105 against 135, 4096 rows 1024 tokens (0.5) 102 against 108, 14336 rows
-// 512 / 640 (0.55 of two) / 1024 / 1400 / 2048 tokens 130 / 219 / 235 / 331 / 443 against 167 / 244 / 302 /
-// 381 / 533; Q5_K 14336 rows 512 / 1024 tokens 144 / 249 against 179 / 332; below half, 2048 rows x 8192
-// 1400 tokens (0.34) 186 against 163, 1300 rows 1400 tokens (0.22) 99 against 70. Rows of fewer than four
-// blocks, shorter than any model's, stay on the 128 x 128 tiles, whose tests hold them there.
+// 384 tokens (0.5 of one round) 105 against 135, 4096 rows 1024 tokens (0.5) 102 against 108, 14336
+// rows 512 / 640 (0.55 of two) / 1024 / 1400 / 2048 tokens 130 / 219 / 235 / 331 / 443 against 167 /
+// 244 / 302 / 381 / 533; Q5_K 14336 rows 512 / 1024 tokens 144 / 249 against 179 / 332; below half,
+// 2048 rows x 8192 1400 tokens (0.34) 186 against 163, 1300 rows 1400 tokens (0.22) 99 against 70. Rows
+// that are no multiple of 4 have their outputs stored one by one. They lose where the 128 x 64 tiles
+// would take a Q4_K launch of one token tile (45686 x 2048, 107 tokens 88 against 82; 38196 rows, 124
+// tokens 74 against 80), and below 1536 columns in two or three rounds the last of which has less than
+// half its tiles (x 1024 columns, Q4_K 70559 rows 215 tokens (2.16 tiles a CU) 130 against 119, 59211
+// rows 179 tokens (1.81) 90 against 95; Q5_K 31423 rows 292 tokens (1.44) 86 against 80; 14336 x 1280,
+// 618 tokens (1.09) 79 against 90). Rows of fewer than four blocks were not swept.
 static bool split_better(const WeightDev &w, const jk_act_q8 &a, long rows) {
     if (!gemm_split_ok(w, a) || w.cols < 1024) return false;
     const long ncu = cu_count(), m = (long)a.m;
-    const long rounds = ((rows + 255) / 256 * ((m + 127) / 128) + ncu - 1) / ncu;
+    const long tm = (m + 127) / 128, tiles = (rows + 255) / 256 * tm, rounds = (tiles + ncu - 1) / ncu;
+    if (rows % 4 != 0) {
+        if (w.quant == JK_Q4_K && tm == 1 && 2 * ((rows + 127) / 128) < 3 * ncu) return false;
+        if (w.cols < 1536 && rounds > 1 && rounds <= 3 && 2 * (tiles - (rounds - 1) * ncu) < ncu) return false;
+    }
     return 2 * rows * m >= 256 * 128 * ncu * rounds;
 }
 

@@ -260,6 +260,7 @@ jk_status launch_gemm_repacked(hipStream_t s, const WeightDev &w, const jk_act_q
 // The repacked GEMM for launches with few output tiles (jk_gemm_few.hip): the weights and activations
 // it takes, and the launch (bit-identical to the tiled kernels).
 bool gemm_few_ok(const WeightDev &w, const jk_act_q8 &a);
+long gemm_few_workgroups(int quant, long rows, long m, long ncu);  // of that launch
 jk_status launch_gemm_few(hipStream_t s, const WeightDev &w, const jk_act_q8 &a, float *y, int r0, int r1, long ncu,
                           bool tol);
 // The tolerance-mode GEMM of Q4_K and Q5_K with the group scales in f16 operands (jk_gemm_split.hip).

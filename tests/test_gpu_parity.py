@@ -197,8 +197,9 @@ def test_subln_absmax_sizes(gpu, k, offset):
 @pytest.mark.parametrize("k", [5, 64, 256, 257, 1024, 1025, 2051, 3072, 4096, 4100, 7169])
 def test_absmax_rows_and_sizes(gpu, m, k):
     """Both absmax quantizers at few rows, more rows than CUs and more than four times as many, on both sides of
-    the row lengths where the launch changes, aligned and not, in one piece and several: normal rows, rows of bf16 values (whose squares lie between two
-    ulps of the running sum again and again) and mostly-zero rows, equal to the oracle."""
+    the row lengths where the launch changes, aligned and not, in one piece and several: normal rows, rows of
+    bf16 values (whose squares lie between two ulps of the running sum again and again) and mostly-zero
+    rows, equal to the oracle."""
     torch = gpu
     rng = np.random.default_rng(m + k)
     x = rng.standard_normal((m, k)).astype(np.float32)
@@ -650,9 +651,10 @@ def test_gemv_repacked_one_or_two_tokens(gpu, quant, m, rows, cols):
 @pytest.mark.parametrize("m", [500, 250, 128, 30])
 def test_gemm_tile_shapes(gpu, quant, m):
     """8200 rows: 500 tokens launch 128x64 tiles, 250 tokens 64x64, 128 tokens 32x32, 30
-    tokens the single-wave 32x16 tiles (32x32 for Q6_K): the launcher takes the largest tile
-    that gives 256 CUs two workgroups each. The last row tile and token tile are partial.
-    Oracle on row windows."""
+    tokens the single-wave 32x16 tiles (32x32 for the 16-element-group formats): the launcher takes the
+    largest tile that gives 256 CUs two workgroups each. Q4_0, Q8_0, Q4_K, Q5_K and Q6_K run the few-tile
+    kernel at most of these counts (test_gemm_live_tiles has their tiles). The last row tile and token
+    tile are partial. Oracle on row windows."""
     torch = gpu
     rows, cols = 8200, 512
     raw = synth.random_weights(quant, rows, cols, seed=m + 3 * quant, specials=True)
@@ -663,6 +665,40 @@ def test_gemm_tile_shapes(gpu, quant, m):
     for r0 in (0, 4091, rows - 45):
         ref = O.gemm_repacked(quant, [rows, cols], raw, rows, cols, act, r0, r0 + 45)
         assert same_bits(got[:, r0:r0 + 45], ref), (r0, mismatch(got[:, r0:r0 + 45], ref))
+
+
+# (format, tokens, rows, columns, launch): the tiles that are left to the tiled kernels in the formats of the
+# few-tile one, on 256 CUs (480 columns: an odd number of 32-element blocks, which it does not take)
+LIVE_TILES = [(Q8_0, 250, 8200, 512, "64x64"), (Q8_0, 66, 9274, 512, "32x32"), (Q4_0, 170, 14300, 512, "64x64"),
+              (Q4_0, 100, 14300, 2048, "32x32"), (Q4_K, 200, 14300, 512, "64x64"), (Q5_K, 170, 14300, 512, "64x64"),
+              (Q5_K, 100, 14300, 512, "32x32"), (Q6_K, 170, 14300, 512, "64x64"), (Q6_K, 100, 14300, 512, "32x32"),
+              (Q8_0, 30, 8000, 480, "16"), (Q4_0, 30, 8000, 480, "16")]
+
+
+@pytest.mark.parametrize("quant,m,rows,cols,launch", LIVE_TILES)
+def test_gemm_live_tiles(gpu, quant, m, rows, cols, launch):
+    """The tiled bit-exact launches that Q4_0, Q8_0, Q4_K, Q5_K and Q6_K still take, each confirmed by the launch
+    plan: partial last row and token tiles, weights with special scales, NaN activations; oracle on row windows
+    (the first, a middle and the partial last tile), a row slice equal to the full call. In tolerance
+    mode the 64 x 64 launches are the same kernel (Q6_K: its K split)."""
+    torch = gpu
+    raw = synth.random_weights(quant, rows, cols, seed=m + 3 * quant, specials=True)
+    rng = np.random.default_rng(m)
+    x = rng.standard_normal((m, cols)).astype(np.float32)
+    x[rng.random((m, cols)) < 0.002] = np.nan
+    w = jk.Weight(jk.TensorView("w", quant, [rows, cols], raw), rows, cols)
+    kernel = "gemm16_kernel" if launch == "16" else f"gemm_repacked_kernel<{launch}>"
+    storage, act = gpu_act(torch, x, m, cols)
+    assert jk.gemm_plan(w, act, 0, rows, False) == kernel
+    got = gpu_gemm(torch, w, x, m)
+    oact = O.ActQ8(x, m, cols)
+    for r0 in (0, rows // 2, rows - 45):
+        ref = O.gemm_repacked(quant, [rows, cols], raw, rows, cols, oact, r0, r0 + 45)
+        assert same_bits(got[:, r0:r0 + 45], ref), (r0, mismatch(got[:, r0:r0 + 45], ref))
+    assert same_bits(gpu_gemm(torch, w, x, m, 3, rows - 5), got[:, 3:rows - 5])
+    if launch == "64x64" and quant != Q6_K:
+        assert same_bits(gpu_gemm_tol(torch, w, x, m, expect=kernel), got)
+    w.free()
 
 
 def gpu_gemm_tol(torch, w, x, m, r0=0, r1=None, expect=None):
@@ -741,8 +777,8 @@ def test_gemm_q8_0_prefill_full_matrix_vs_exact_product(gpu):
 @pytest.mark.parametrize("quant", ALL_FORMATS)
 @pytest.mark.parametrize("m", [500, 250, 128, 30])
 def test_gemm_tol_tile_shapes(gpu, quant, m):
-    """Tolerance-mode GEMM on every format and tile shape (8200 rows: 128x64, 64x64 and 32x32
-    tiles; partial last row and token tiles; weights with special scales): within 1e-5 of each
+    """Tolerance-mode GEMM on every format (8200 rows: 128x64 and 64x64 tiles and the K split, or the few-tile
+    kernel in its formats; partial last row and token tiles; weights with special scales): within 1e-5 of each
     token's output-row L2 norm of the oracle on row windows and of the bit-exact GPU output over
     the whole matrix, and row slices equal to the full call."""
     torch = gpu
@@ -864,7 +900,7 @@ def test_gemm_q8_0_exact_staged_tiles(gpu):
 
 
 FEW_SHAPES = [(3, 37, 512), (16, 100, 2816), (4, 1003, 768), (5, 4201, 512), (33, 4200, 768), (40, 8205, 512),
-              (47, 14000, 512), (61, 12003, 768), (77, 8500, 512)]
+              (47, 14000, 512), (61, 12003, 768), (81, 8100, 512)]
 
 
 @pytest.mark.parametrize("quant", [Q8_0, Q4_0, Q4_K, Q5_K, Q6_K])
@@ -1045,7 +1081,9 @@ def test_gemm_tol_split_k(gpu, quant, m, chunks):
     """Tolerance-mode GEMM of a few tokens, where K is split over the waves of a workgroup: K of
     1 to 13 chunks of 128 (waves with no chunk, with one more chunk than the others), 32- and
     64-token tiles with a partial last one (Q6_K / Q3_K: 64-token tiles, the two 16-element groups of
-    a step combined in integers), 200 rows (a partial last row tile) and a row slice.
+    a step combined in integers), 200 rows (a partial last row tile) and a row slice. (Q4_0, Q8_0, Q4_K,
+    Q5_K and Q6_K run the few-tile kernel at these shapes, test_gemm_tol_split_k_many_tiles has their
+    splits.)
     Held within 1e-5 of each token's output-row L2 norm of the bit-exact GPU output over the whole
     matrix and of the oracle on a row window."""
     torch = gpu
@@ -1065,6 +1103,27 @@ def test_gemm_tol_split_k(gpu, quant, m, chunks):
     assert np.all(np.abs(tol[:, 150:200] - ref).max(axis=1) <= 1e-5 * norms)
     sl = gpu_gemm_tol(torch, w, x, m, 5, 171)
     assert_within_row_norm(sl, exact[:, 5:171])
+    w.free()
+
+
+@pytest.mark.parametrize("quant", [Q8_0, Q4_0, Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("m,rows,chunks", [(17, 9000, 6), (33, 13000, 4), (64, 4200, 14), (100, 2500, 10)])
+def test_gemm_tol_split_k_many_tiles(gpu, quant, m, rows, chunks):
+    """The K-split tolerance launches of the formats that the few-tile kernel takes too, at more 16 x 16 tiles
+    than it has the better of, confirmed by the launch plan: 32- and 64-token tiles with a partial last one,
+    a partial last row tile; the bars of test_gemm_tol_split_k."""
+    torch = gpu
+    cols = 128 * chunks
+    raw = synth.random_weights(quant, rows, cols, seed=7 * m + chunks + quant, specials=True)
+    x = np.random.default_rng(m + chunks).standard_normal((m, cols)).astype(np.float32)
+    w = jk.Weight(jk.TensorView("w", quant, [rows, cols], raw), rows, cols)
+    exact = gpu_gemm(torch, w, x, m)
+    tokens = 32 if m <= 32 and quant != Q6_K else 64
+    tol = gpu_gemm_tol(torch, w, x, m, expect=f"gemm_tol_splitk_kernel<{tokens} tokens>")
+    assert_within_row_norm(tol, exact)
+    ref = O.gemm_repacked(quant, [rows, cols], raw, rows, cols, O.ActQ8(x, m, cols), rows - 50, rows)
+    assert same_bits(exact[:, rows - 50:], ref)
+    assert_within_row_norm(gpu_gemm_tol(torch, w, x, m, 5, rows - 2), exact[:, 5:rows - 2])
     w.free()
 
 
