@@ -493,10 +493,17 @@ static jk_status launch_few_q(hipStream_t s, const WeightDev &w, const jk_act_q8
         else return launch_few_t<Q, 2, 1, 4, 4>(s, w, a, y, r0, r1, tol);
     case kFew2x2x4: return launch_few_t<Q, 2, 2, 4, 4>(s, w, a, y, r0, r1, tol);
     case kFew2x2x2: return launch_few_t<Q, 2, 2, 2, 2>(s, w, a, y, r0, r1, tol);
-    case kFew4x2: return launch_few_t<Q, 4, 2, 2, 1>(s, w, a, y, r0, r1, tol);
-    case kFew4x3: return launch_few_t<Q, 4, 3, 2, 1>(s, w, a, y, r0, r1, tol);
-    default: return launch_few_t<Q, 4, 4, 2, 1>(s, w, a, y, r0, r1, tol);
+    case kFew4x2:
+        if constexpr (Q != JK_Q6_K && Q != JK_Q8_0) return launch_few_t<Q, 4, 2, 2, 1>(s, w, a, y, r0, r1, tol);
+        break;
+    case kFew4x3:
+        if constexpr (Q != JK_Q6_K) return launch_few_t<Q, 4, 3, 2, 1>(s, w, a, y, r0, r1, tol);
+        break;
+    default:
+        if constexpr (Q != JK_Q6_K) return launch_few_t<Q, 4, 4, 2, 1>(s, w, a, y, r0, r1, tol);
+        break;
     }
+    return fail(JK_DEVICE_ERROR, "gemm: no few-tile launch of quant %d", w.quant);  // (few_shape gives none of these)
 }
 
 bool gemm_few_ok(const WeightDev &w, const jk_act_q8 &a) {
