@@ -327,19 +327,27 @@ jk_status jk_vec_dot_f32_tol(jk_stream s, const jk_weight *w, const float *x, si
 jk_status jk_gemm_repacked(jk_stream s, const jk_weight *w, const jk_act_q8 *act, float *y,
                            size_t y_len, size_t row_begin, size_t row_end);
 /* gemm_repacked_rows (repack.rs:4087-4094) in tolerance mode: the same arguments, validation and
- * errors as jk_gemm_repacked, with each scale group's exact integer partial applied by one fused
- * multiply-add (acc = fma(partial, xs * ws, acc); formats with mins add -(xsum * wm) as one more
- * rounded step) instead of the reference's separately rounded product and sum. Every output is
+ * errors as jk_gemm_repacked, with each scale group's exact integer partial applied by fused
+ * multiply-adds instead of the reference's separately rounded product and sum. Every output is
  * within 1e-5 of its token's output-row L2 norm of the bit-exact result (the tolerance the port
- * is held to for f32 products). From 1.5 128 x 128 tiles per CU on (14336 rows: 448 tokens), the
- * 32-element-group formats run larger tiles with fewer VALU operations per scale group, about
- * 1.2x the throughput of jk_gemm_repacked; Q8_0 there applies each group as
- * fma(B + partial, ws * xs, acc - B * ws * xs) with B = 1.5 * 2^23 (the second product accumulated on
- * the matrix core), so a scale product |ws * xs| above 2^104 can overflow to infinity where the
- * bit-exact call stays finite. Q6_K and Q3_K combine a step's two 16-element groups in integers;
- * Q2_K, and launches where the bit-exact tiles measured faster, run the bit-exact kernels (whose
- * results meet the bar by definition). No reference function has this rounding: it is the
- * bit-exact call's alternative. */
+ * is held to for f32 products). No reference function has this rounding: it is the bit-exact
+ * call's alternative. By launch, whichever measured fastest:
+ * - in general acc = fma(partial, xs * ws, acc), formats with mins adding -(xsum * wm) as one more
+ *   rounded step. With few output tiles K is split: each of up to eight waves (Q4_0, Q8_0, Q4_K,
+ *   Q5_K, Q6_K: four accumulators a wave) adds its groups, and their sums are added at the end.
+ * - From 1.5 128 x 128 tiles per CU on (14336 rows: 448 tokens), the 32-element-group formats run
+ *   larger tiles with fewer VALU operations per scale group; Q8_0 there applies each group as
+ *   fma(B + partial, ws * xs, acc - B * ws * xs) with B = 1.5 * 2^23 (the second product accumulated on
+ *   the matrix core), so a scale product |ws * xs| above 2^104 can overflow to infinity where the
+ *   bit-exact call stays finite. Q6_K and Q3_K combine a step's two 16-element groups in integers.
+ * - Q4_K and Q5_K from 1024 columns where 256 x 128 tiles, one per CU, are at least half full: the
+ *   6-bit scales sc and mins mn are multiplied exactly, and d and dmin once per 256-element block:
+ *   part = fma(partial * sc, xs, part) over its groups, acc = fma(d, part, acc), then
+ *   acc = fma(-dmin, sum(xsum * mn), acc) (xsum to 24 bits). Both block sums stay finite for every
+ *   finite xs and xsum; an output whose terms cancel within a factor of 16 of f32's largest value
+ *   can overflow where the bit-exact call's order of additions does not.
+ * - Q2_K, and launches where the bit-exact tiles measured faster, run the bit-exact kernels (whose
+ *   results meet the bar by definition). */
 jk_status jk_gemm_repacked_tol(jk_stream s, const jk_weight *w, const jk_act_q8 *act, float *y,
                                size_t y_len, size_t row_begin, size_t row_end);
 /* gemv_repacked_view_rows (repack.rs:4045-4061): requires act->m == 1. */

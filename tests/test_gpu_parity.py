@@ -1018,6 +1018,50 @@ def test_gemm_split_range(gpu, quant):
     w.free()
 
 
+def k_quant_f64(quant, raw, rows, cols):
+    """Q4_K / Q5_K weights in 64 bits: the values without their mins, and the mins per 32 elements."""
+    b = np.frombuffer(np.asarray(raw).tobytes(), np.uint8).reshape(rows, cols // 256, jk.BLOCK_BYTES[quant])
+    d, dm = (b[..., i:i + 2].copy().view(np.float16)[..., 0].astype(np.float64) for i in (0, 2))
+    lo, hi, mix = b[..., 4:8], b[..., 8:12], b[..., 12:16]
+    sc = np.concatenate([lo & 63, (mix & 15) | (lo >> 6 << 4)], -1).astype(np.float64)
+    mn = np.concatenate([hi & 63, (mix >> 4) | (hi >> 6 << 4)], -1).astype(np.float64)
+    qs = b[..., -128:].reshape(rows, -1, 4, 1, 32)
+    q = np.concatenate([qs & 15, qs >> 4], 3).reshape(rows, -1, 8, 32).astype(np.float64)
+    if quant == Q5_K:
+        q += 16 * ((b[..., 16:48][:, :, None] >> np.arange(8, dtype=np.uint8)[:, None]) & 1)
+    return (q * (d[..., None] * sc)[..., None]).reshape(rows, cols), (dm[..., None] * mn).reshape(rows, cols // 32)
+
+
+@pytest.mark.parametrize("quant", [Q4_K, Q5_K])
+@pytest.mark.parametrize("m,rows,expect", [(300, 14343, "gemm_split_kernel"), (50, 3000, "gemm_few_kernel<tolerance>")])
+@pytest.mark.parametrize("mins", [False, True])
+def test_gemm_tol_precision(gpu, quant, m, rows, expect, mins):
+    """The tolerance kernels' rounding: within 1e-6 (2-norm) of the float64 product of the same quantized
+    operands (128 group additions, each rounded by up to 2^-24 of a partial sum: sqrt(128) 2^-24 = 6.7e-7); also
+    where the mins and the activations' sums make up most of each output (sums of which only 16 of 24
+    bits were kept would be 4e-6 off)."""
+    torch = gpu
+    cols = 4096
+    raw = synth.gguf_weights(quant, rows, cols, seed=quant + m)
+    rng = np.random.default_rng(m)
+    x = rng.standard_normal((m, cols)) * np.exp2(rng.integers(-3, 4, (m, 1)))
+    if mins:
+        raw.reshape(-1, jk.BLOCK_BYTES[quant])[:, 0:2] = np.float16(1e-4).view(np.uint16).reshape(1, 1).view(np.uint8)
+        x = np.abs(x)
+    x = x.astype(np.float32)
+    w = jk.Weight(jk.TensorView("w", quant, [rows, cols], raw), rows, cols)
+    got = gpu_gemm_tol(torch, w, x, m, expect=expect).astype(np.float64)
+    act = O.ActQ8(x, m, cols)
+    xq = (act.qs.astype(np.float64).reshape(m, -1, 32) * act.scales.astype(np.float64)[..., None]).reshape(m, cols)
+    for r0, r1 in ((0, 300), (rows - 300, rows)):
+        wq, mn = k_quant_f64(quant, raw.reshape(rows, -1)[r0:r1], r1 - r0, cols)
+        ref = xq @ wq.T - act.sums.astype(np.float64) @ mn.T
+        err = np.linalg.norm(got[:, r0:r1] - ref) / np.linalg.norm(ref)
+        print(f"gemm tol {quant} {expect} mins {mins} rows {r0}..{r1}: {err:.2e}")
+        assert err < 1e-6
+    w.free()
+
+
 TOL128_FORMATS = [Q8_0, Q4_0, Q5_0, Q4_1, Q5_1, IQ4_NL, Q4_K, Q5_K, TQ2_0, I2_S]
 
 
