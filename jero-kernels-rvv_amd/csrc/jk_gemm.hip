@@ -2170,7 +2170,8 @@ static bool few_better(const WeightDev &w, const jk_act_q8 &a, long rows, bool t
 // tokens 74 against 80), and below 1536 columns in two or three rounds the last of which has less than
 // half its tiles (x 1024 columns, Q4_K 70559 rows 215 tokens (2.16 tiles a CU) 130 against 119, 59211
 // rows 179 tokens (1.81) 90 against 95; Q5_K 31423 rows 292 tokens (1.44) 86 against 80; 14336 x 1280,
-// 618 tokens (1.09) 79 against 90). Rows of fewer than four blocks were not swept.
+// 618 tokens (1.09) 79 against 90). Rows of fewer than four blocks, shorter than any model's, stay on
+// the 128 x 128 tiles, which the tests check at 512 columns (14336 x 512, 512 tokens 26 against 38).
 static bool split_better(const WeightDev &w, const jk_act_q8 &a, long rows) {
     if (!gemm_split_ok(w, a) || w.cols < 1024) return false;
     const long ncu = cu_count(), m = (long)a.m;

@@ -19,11 +19,13 @@
 // scale products run on all the waves; only the additions are a chain. In tolerance mode the order
 // is free: each wave keeps sums of its own (one fused multiply-add per group), added at the end.
 //
-// What bounds it (counters at 4096 x 4096, 64 tokens): the chain's hand-over at few tiles, and from
-// about eight tiles per CU the VALU -- some 130 of 215 instructions a unit and tile are the four
-// operations per output and group that the recipe takes (Q4_K) -- next to which loads straight
-// from global memory in the operands' layout (64 lines a load) had kept the address unit busy 80%
-// of the time.
+// What bounds it: the chain's hand-over at few tiles (Q6_K 4096 x 14336 at 4 tokens: VALU busy 50% of the
+// cycles, a wave waiting 44% of its time; 24 us), and from about eight tiles per CU the VALU (512 tokens: 99%;
+// Q4_0 11008 x 4096 at 150 tokens in tolerance mode 74%, and 29% f32 and integer MFMAs, of which the f32 ones
+// stall it). Of its instructions a unit and tile some 130 in 215 are the four operations per output and group
+// that the recipe takes (Q4_K); unpacking, swapping and scaling the operands for a single 16 x 16 tile are
+// the rest. Next to these, loads straight from global memory in the operands' layout (64 lines a load) had
+// kept the address unit busy 80% of the time.
 //
 // Operands: lane l holds weight row (or token) l % 16 and part kq = l / 16 of K. For a pair of
 // 32-element groups lane kq reads 16 bytes -- piece kq % 2 of group kq / 2 of the pair -- and

@@ -19,10 +19,16 @@
 // into one of two LDS stages a 256-element block ahead, activations through registers a 64-element
 // quarter ahead, converted to f16 once per workgroup; a wave unpacks the weights that it multiplies.
 //
-// What bounds it: the VALU, with one multiply-add per output and group (16 an MFMA pair) and about a third
-// as much again for unpacking, converting and the blocks' ends; f16 MFMAs run under it. 14336 x 4096,
-// Q4_K: 2048 tokens 443 us (543 TOPS) against 533 us on the 128 x 128 tiles, 512 tokens 130 against 167 us,
-// and the error against 64 bits 1.7e-7 against 3.1e-7. Timed with work left out: loading no weights 408 us.
+// What bounds it: each wave's own chain, LDS read -> MFMA -> multiply-adds, one tile deep, at two waves a
+// SIMD and a workgroup barrier every 64 elements. Counted at 14336 x 4096, 2048 tokens: the VALU is busy 53%
+// of the cycles (2.2 instructions per output and group, of which the multiply-add is one; unpacking,
+// converting and the blocks' ends are the rest), the matrix cores 27%, the LDS 39% (a third of it bank
+// conflicts), and a wave waits a third of its time. 14336 x 4096, Q4_K: 2048 tokens 443 us (543 TOPS) against
+// 533 us on the 128 x 128 tiles (launched back to back; 485 us and more under a profiler), 512 tokens 130
+// against 167 us, and the error against 64 bits 1.7e-7 against 3.1e-7. Timed with work left out: loading no
+// weights 408 us. (The weights' loads are asm that the compiler does not count, so its wait for the
+// activations' loads, two tiles into a quarter, waits for the quarter's weights too: more than needed, never
+// less. The explicit wait at a block's end is for all of them.)
 // Also tried, both with the activation scales in the operands (x * xs as two f16 numbers, no multiply-add
 // per group): 552 us, the conversion and twice the MFMAs taking more than they save, and 565 us with its
 // MFMAs and VALU work interleaved by hand. What made it fast: each tile's sum pinned where it is added (the
