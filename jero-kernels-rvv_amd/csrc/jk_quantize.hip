@@ -290,8 +290,8 @@ __global__ __launch_bounds__(NT) void absmax_i8_kernel(const float *__restrict__
 // approximate prefix can lie a few ulps below the end of the thread before it, put together in another
 // order, and fall back into the binade below); where a check fails, or with too many elements outside
 // the rule, the first wave adds the whole row in order. Normal rows of 2560 and 6912 have 12 and 14 such
-// elements, of f32 and of bf16 values alike: 7.6 and 10.8 us a launch (with every tie added one by one
-// 8.2 and 11 us, and for bf16 values, 325 and 726 ties, 60 and 152 us). What bounds it now: the scans'
+// elements, of f32 and of bf16 values alike: 7.6 and 9.3 us a launch (with every tie added one by one
+// 8.0 and 10 us, and for bf16 values, 325 and 726 ties, 59 and 151 us). What bounds it now: the scans'
 // cross-lane steps, the elements added one by one (a scalar round trip each) and three passes over the row.
 constexpr int kAbsThreads = 1024;
 constexpr int kSqSerial = 256;    // pieces up to this length are added one by one
@@ -395,15 +395,16 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
     const float waves = scan_add<false>(lane < NW ? L.part[lane] : 0.0f);
     const float before_wave = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(waves), max(wave - 1, 0)));
     const float pre = acc0 + (wave > 0 ? before_wave : 0.0f) + (incl - part);  // approximate sum before the thread
-    // element i after an approximate sum p: its binade, whether it goes by the rule, and its increments
-    auto element = [&](int i, float p, uint32_t &eb, bool &ok) {
+    // adds element i, after an approximate sum p, to a run: its binade, and whether it goes by the rule
+    auto element = [&](int i, float p, SumRun &run, uint32_t &eb) {
         eb = __float_as_uint(p * 0.99998f) >> 23;
         const uint32_t ee = __float_as_uint((p + v[i]) * 1.00002f) >> 23;
         const float to_ulp = __uint_as_float((277u - min(max(eb, 30u), 220u)) << 23);  // 1 / u, a power of two
         const float w = v[i] * to_ulp, fl = floorf(w), fr = w - fl;
-        ok = eb == ee && eb >= 30 && eb <= 220 && w < 16777216.0f;
-        const int b = (int)fl, up = fr > 0.5f, tie = fr == 0.5f;
-        return ok ? SumRun{b + (up | (tie & b)), b + (up | (tie & ~b))} : SumRun{0, 0};
+        const int r = (int)fl + (fr > 0.5f), tie = fr == 0.5f;
+        const int a = run.even + r, b = run.odd + r;  // (a tie: one more if that makes the sum even)
+        run = {a + (a & tie), b + (~b & tie)};
+        return eb == ee && eb >= 30 && eb <= 220 && w < 16777216.0f;
     };
     uint32_t events = 0;
     SumRun run = {0, 0};  // since the last event
@@ -413,12 +414,9 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         uint32_t eb;
-        bool ok;
-        const SumRun r = element(i, p, eb, ok);
+        const bool ok = element(i, p, run, eb), live = lo + i < n;  // (past the end: zeros, which add nothing)
         p += v[i];
-        const bool live = lo + i < n;
-        const SumRun next = run_then(run, r);
-        run = live ? (ok ? next : SumRun{0, 0}) : run;
+        if (live && !ok) run = {0, 0};
         events |= (uint32_t)(live && !ok) << i;
         if (lo + i == n - 1) L.tail_eb = (int)eb;
         if (i == 0) first = live ? eb : kNoRun;
@@ -449,16 +447,15 @@ __device__ __forceinline__ float parallel_ordered_sum(float acc0, const float *s
         p = pre;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
+            const SumRun before = run;
             uint32_t eb;
-            bool ok;
-            const SumRun r = element(i, p, eb, ok);
+            element(i, p, run, eb);
             p += v[i];
             const bool event = (events >> i) & 1u;
             if (event && ci < kSqEvents)
-                L.ev[ci] = make_int4((lo + i) << 9 | (int)eb, run.even, run.odd, __float_as_int(v[i]));
+                L.ev[ci] = make_int4((lo + i) << 9 | (int)eb, before.even, before.odd, __float_as_int(v[i]));
             ci += event;
-            const SumRun next = run_then(run, r);
-            run = event ? SumRun{0, 0} : next;
+            if (event) run = {0, 0};
         }
     }
     __syncthreads();
