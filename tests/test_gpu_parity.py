@@ -923,6 +923,8 @@ def test_gemm_few_tiles(gpu, quant, m, rows, cols):
     w = jk.Weight(jk.TensorView("w", quant, [rows, cols], raw), rows, cols)
     storage, act = gpu_act(torch, x, m, cols)
     assert jk.gemm_plan(w, act, 0, rows, False) == "gemm_few_kernel"
+    if (rows + 15) // 16 * ((m + 15) // 16) <= 512:  # two 16 x 16 tiles per CU
+        assert jk.gemm_plan(w, act, 0, rows, True) == "gemm_few_kernel<tolerance>"
     got = gpu_gemm(torch, w, x, m)
     oact = O.ActQ8(x, m, cols)
     for r0, r1 in ((0, 33), (rows // 2, rows // 2 + 20), (rows - 35, rows)):
